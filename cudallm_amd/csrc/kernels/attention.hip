@@ -3,13 +3,14 @@
 // Semantics (what is computed, which buffers change) follow the reference:
 //   rope_kv fused / unfused      src/kernels/rope_kv.cu:10-79  (pairs (i, i+hd/2), angle fp32(pos)*inv_freq[i],
 //                                fused leaves the k slice of qkv unrotated)
-//   split-K partial + LSE merge  src/kernels/attention_opt.cu:17-134 (scale 0.125, 128-token splits, splits at or
-//                                past ctx exit at once so the grid is fixed and graph-capturable, merge in split order)
+//   split-K + LSE merge          src/kernels/attention_opt.cu:17-134 (scale 0.125, splits at or past ctx exit at once so
+//                                the grid is fixed and graph-capturable)
 //   naive                        src/kernels/attention_naive.cu:18-81 (one workgroup per query head)
-// The gfx950 layout is this file's: a 256-thread workgroup = 4 waves = the 4 query heads of one
-// kv head, each lane scores two tokens (lane, lane+64) with the query held in VGPRs, and each lane
-// owns one of the 64 output dimensions for the p.V accumulation.
+// How the split-K kernel divides the work is this file's own, described at the kernel.
+#include <algorithm>
 #include <array>
+#include <atomic>
+#include <cfloat>
 #include <mutex>
 
 #include "../kernels.h"
@@ -81,100 +82,325 @@ __global__ void __launch_bounds__(256) kv_write_kernel(const float* qkv, uint16_
     cache[(static_cast<size_t>(head) * max_seq + *d_pos) * hd + d] = float_to_half_bits(qkv[nh * hd + t]);
 }
 
-// grid (nkv, max_seq/128), block 256.  LDS: K tile with one padding dword per row so lane j's row
-// reads hit distinct banks, V tile unpadded (lanes read consecutive halves), p per head.
-__global__ void __launch_bounds__(256) attn_partial_kernel(const float* q, const uint16_t* kc, const uint16_t* vc,
-                                                           const int* d_pos, float* part_o, float* part_ml, int max_seq) {
-    __shared__ uint32_t Ks[kAttnChunk][kHd / 2 + 1];
-    __shared__ u32x4 Vs[kAttnChunk][kHd / 8];
-    __shared__ float ps[kGroup][kAttnChunk];
+// ---- split-K attention -------------------------------------------------------------------------------
+//
+// One kernel.  Bound by the K and V bytes at long contexts, by latency at short ones.  A wave takes whole 32-token
+// tiles: lane (g, c) = (lane / 8, lane % 8) loads 16 bytes, columns 8c .. 8c + 7, of tokens g, g + 8, g + 16 and g + 24,
+// so every load instruction reads 1 KiB of consecutive cache rows straight into registers (no LDS staging), and the next
+// tile's 8 KiB are in flight while this one is multiplied.  All 4 query heads of the kv head run on the same registers:
+// 8 mixed-precision FMAs per head and token, summed over the 8 column lanes by DPP.  Each token phase g keeps its own
+// running softmax (m, l, o), so the loop exchanges nothing between phases; they are merged once, at the wave's end,
+// then the workgroup's 8 waves in LDS.
+//
+// A kv head's tiles are dealt over its splits' waves as evenly as whole tiles allow, with only as many splits as give
+// every wave a tile: up to 256 tokens are one workgroup, which writes the output.  With more, each split publishes its
+// (o, m, l) as tagged words (value and tag in one 64-bit word, so a word that carries the tag carries the value) and the
+// last split's workgroup polls them and writes the output: one store-to-load hop instead of a second launch.
+//  * The workgroups it waits for have smaller indices and wait for nothing, so they have been dispatched before it and
+//    always finish.  The wait is bounded besides; should it run out, the outputs are NaN.
+//  * The tag is a NaN pattern with the launch's number, which scratch memory does not hold by accident, and the words
+//    are zeroed as they are consumed, so a replayed launch (same number) never meets its own earlier words.
+// Measured on MI355X, 8 kv heads, one call in a replayed graph of 16 (2 at 131071), before (128 tokens per workgroup
+// staged in LDS, a second kernel merging the splits one after the other) and now: 100 tokens 6.5 -> 5.3 us, 1000
+// 9.7 -> 7.7, 4000 18.4 -> 8.8, 8000 28.0 -> 11.0, 131071 375 -> 52 (5.1 TB/s).
+// Workgroups in all: one per CU (2 waves per SIMD).  With workgroups of half the size, 512 measured 57 against 52 us
+// at 131071 tokens and 12.7 against 11.4 at 8000, 128 measured 82 and 11.7.
+constexpr int kSplitBlocks = 256;
+constexpr int kMaxSplits = 64;     // splits of one kv head
+constexpr int kWaves = 8;          // per workgroup
+constexpr int kTile = 32;
+constexpr int kTileRows = kTile / 8;
+constexpr float kScore2 = 0.125f * 1.4426950408889634f;  // score scale times log2(e)
 
-    const int ctx = *d_pos + 1;
-    const int kvh = blockIdx.x, split = blockIdx.y;
-    const int t0 = split * kAttnChunk;
-    if (t0 >= ctx) return;
-    const int n = min(kAttnChunk, ctx - t0);
-    const int tid = threadIdx.x, w = tid / kWave, lane = tid % kWave;
+struct KvTile {
+    u32x4 k[kTileRows], v[kTileRows];
+};
 
-    const uint16_t* Kg = kc + (static_cast<size_t>(kvh) * max_seq + t0) * kHd;
-    const uint16_t* Vg = vc + (static_cast<size_t>(kvh) * max_seq + t0) * kHd;
-    for (int idx = tid; idx < n * 8; idx += 256) {
-        const int t = idx / 8, c = idx % 8;
-        const u32x4 kv = *reinterpret_cast<const u32x4*>(Kg + t * kHd + c * 8);
-        Ks[t][c * 4 + 0] = kv[0];
-        Ks[t][c * 4 + 1] = kv[1];
-        Ks[t][c * 4 + 2] = kv[2];
-        Ks[t][c * 4 + 3] = kv[3];
-        Vs[t][c] = *reinterpret_cast<const u32x4*>(Vg + t * kHd + c * 8);
-    }
-    const int h = kvh * kGroup + w;
-    float qr[kHd];
-#pragma unroll
-    for (int d = 0; d < kHd; d += 4) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(q + h * kHd + d);
-        qr[d] = v[0];
-        qr[d + 1] = v[1];
-        qr[d + 2] = v[2];
-        qr[d + 3] = v[3];
-    }
-    __syncthreads();
+// The running softmax of one token phase: m, l and the lane's 8 output columns for each of the 4 heads, in powers of
+// two: m is the largest score times log2(e), a weight is exp2(score log2(e) - m) from one FMA on the raw dot product.
+// m starts at the lowest float, not -inf, so that a score of -inf (a cached -inf) weighs exp2(-inf) = 0 and not NaN.
+struct Running {
+    float m[kGroup], l[kGroup], o[kGroup][8];
+};
 
-    float s[2];
+__device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// Sum over the 8 column lanes of a token (every lane gets it).
+__device__ __forceinline__ float sum8(float v) {
+    v += dpp<kDppXor1>(v);
+    v += dpp<kDppXor2>(v);
+    return v + dpp<kDppHalfMirror>(v);
+}
+
+// Maximum and sum over the 8 token phases (lane bits 3, 4, 5).
+__device__ __forceinline__ float phase_max(float v) {
+    v = fmaxf(v, dpp<kDppRor8>(v));
+    return max_lanes_xor<32>(max_lanes_xor<16>(v));
+}
+__device__ __forceinline__ float phase_sum(float v) {
+    v += dpp<kDppRor8>(v);
+    v = sum_lanes_xor<16>(v);
+    return sum_lanes_xor<32>(v);
+}
+
+// One tile: tokens t0 + 8 r + g; those at or past ctx weigh nothing.
+__device__ __forceinline__ void attend(const KvTile& kv, const float (&q)[kGroup][8], Running& st, int t0, int g, int ctx) {
+    float s[kTileRows][kGroup];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int j = lane + kWave * k;
-        if (j < n) {
-            float dot = 0.f;
+    for (int r = 0; r < kTileRows; ++r)
 #pragma unroll
-            for (int d2 = 0; d2 < kHd / 2; ++d2) {
-                const uint32_t kk = Ks[j][d2];
-                dot = fmaf(half_bits_to_float(static_cast<uint16_t>(kk)), qr[2 * d2], dot);
-                dot = fmaf(half_bits_to_float(static_cast<uint16_t>(kk >> 16)), qr[2 * d2 + 1], dot);
+        for (int h = 0; h < kGroup; ++h) {
+            float d = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                d = fmaf(half_bits_to_float(static_cast<uint16_t>(kv.k[r][e])), q[h][2 * e], d);
+                d = fmaf(half_bits_to_float(static_cast<uint16_t>(kv.k[r][e] >> 16)), q[h][2 * e + 1], d);
             }
-            s[k] = 0.125f * dot;
-        } else {
-            s[k] = -INFINITY;
+            s[r][h] = sum8(d);
+            if (t0 + 8 * r + g >= ctx) s[r][h] = -INFINITY;
+        }
+    float m[kGroup];
+    bool moved = false;
+#pragma unroll
+    for (int h = 0; h < kGroup; ++h) {
+        m[h] = st.m[h];
+#pragma unroll
+        for (int r = 0; r < kTileRows; ++r) m[h] = fmaxf(m[h], s[r][h] * kScore2);
+        moved = moved || m[h] > st.m[h];
+    }
+    if (__any(moved)) {  // a new maximum somewhere in the wave: rare after a chunk's first tiles
+#pragma unroll
+        for (int h = 0; h < kGroup; ++h) {
+            const float f = exp2_hw(st.m[h] - m[h]);
+            st.m[h] = m[h];
+            st.l[h] *= f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) st.o[h][e] *= f;
         }
     }
-    const float m = wave_max(fmaxf(s[0], s[1]));
-    const float p0 = lane < n ? expf(s[0] - m) : 0.f;
-    const float p1 = lane + kWave < n ? expf(s[1] - m) : 0.f;
-    const float l = wave_sum(p0 + p1);
-    ps[w][lane] = p0;
-    ps[w][lane + kWave] = p1;
-    __syncthreads();
-
-    // Lane = output dimension d: o_d = sum_j p_j V[j][d].
-    const uint16_t* vrow = reinterpret_cast<const uint16_t*>(&Vs[0][0]);
-    float o = 0.f;
-    for (int j = 0; j < n; ++j) o = fmaf(ps[w][j], half_bits_to_float(vrow[j * kHd + lane]), o);
-    const int n_split = max_seq / kAttnChunk;
-    const size_t slot = static_cast<size_t>(h) * n_split + split;
-    part_o[slot * kHd + lane] = o;
-    if (lane == 0) {
-        part_ml[slot * 2] = m;
-        part_ml[slot * 2 + 1] = l;
+#pragma unroll
+    for (int r = 0; r < kTileRows; ++r) {
+        u32x4 v = kv.v[r];
+        if (t0 + 8 * r + g >= ctx) v = u32x4{0, 0, 0, 0};  // the row loaded in its place may hold an inf
+#pragma unroll
+        for (int h = 0; h < kGroup; ++h) {
+            const float p = exp2_hw(fmaf(s[r][h], kScore2, -m[h]));
+            st.l[h] += p;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                st.o[h][2 * e] = fmaf(p, half_bits_to_float(static_cast<uint16_t>(v[e])), st.o[h][2 * e]);
+                st.o[h][2 * e + 1] = fmaf(p, half_bits_to_float(static_cast<uint16_t>(v[e] >> 16)), st.o[h][2 * e + 1]);
+            }
+        }
     }
 }
 
-// grid nh, block 64: merge the active splits of head h in split order.
-__global__ void __launch_bounds__(64) attn_combine_kernel(const float* part_o, const float* part_ml, const int* d_pos,
-                                                          float* out, int max_seq) {
-    const int h = blockIdx.x, d = threadIdx.x;
-    const int ctx = *d_pos + 1;
-    const int used = (ctx + kAttnChunk - 1) / kAttnChunk;
-    const int n_split = max_seq / kAttnChunk;
-    const float* ml = part_ml + static_cast<size_t>(h) * n_split * 2;
-    const float* po = part_o + static_cast<size_t>(h) * n_split * kHd;
-    float M = -INFINITY;
-    for (int s = 0; s < used; ++s) M = fmaxf(M, ml[2 * s]);
-    float L = 0.f, acc = 0.f;
-    for (int s = 0; s < used; ++s) {
-        const float e = expf(ml[2 * s] - M);
-        L = fmaf(ml[2 * s + 1], e, L);
-        acc = fmaf(po[static_cast<size_t>(s) * kHd + d], e, acc);
+// ---- tagged words -----------------------------------------------------------------------------------
+
+typedef __attribute__((address_space(1))) uint64_t global_u64;
+__device__ __forceinline__ uint64_t tag_load(const uint64_t* p) {
+    return __hip_atomic_load((global_u64*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void tag_store(uint64_t* p, float v, uint32_t tag) {
+    __hip_atomic_store((global_u64*)p, static_cast<uint64_t>(tag) << 32 | __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool has_tag(uint64_t v, uint32_t tag) { return static_cast<uint32_t>(v >> 32) == tag; }
+__device__ __forceinline__ float value_of(uint64_t v) { return __builtin_bit_cast(float, static_cast<uint32_t>(v)); }
+
+constexpr unsigned kPollCap = 1u << 20;  // about a second
+
+// Where the partials of head h's split s lie: o as [h][s][64], then m and l as [h][s][2].
+struct Partials {
+    uint64_t *o, *ml;
+    uint32_t tag;
+};
+
+// The first n (<= used - 1) splits of head h that fall to this wave, s = half, half + 2, ...: their merged (m, l) and the
+// lane's output column.  Up to 16 of them, and all of their (m, l), are in flight at once.
+__device__ __forceinline__ void merge_half(const Partials& p, int h, int splits, int n, int half, int lane, float& m, float& l,
+                                           float& o) {
+    constexpr int kRound = 16;
+    m = -FLT_MAX, l = 0.f, o = 0.f;
+    uint64_t* po = p.o + static_cast<size_t>(h) * splits * kHd + lane;
+    uint64_t* pml = p.ml + static_cast<size_t>(h) * splits * 2;
+    const uint64_t none = static_cast<uint64_t>(p.tag) << 32;
+    for (int s0 = half; s0 < n; s0 += 2 * kRound) {
+        const int sl = s0 + 2 * (lane % kRound);  // the split whose m (lanes 0-15) or l (16-31) this lane polls
+        const bool mine = lane < 2 * kRound && sl < n;
+        uint64_t* const pm = pml + (mine ? 2 * sl + lane / kRound : 0);
+        uint64_t vm = mine ? tag_load(pm) : none, v[kRound];
+#pragma unroll
+        for (int i = 0; i < kRound; ++i) v[i] = s0 + 2 * i < n ? tag_load(po + static_cast<size_t>(s0 + 2 * i) * kHd) : none;
+        for (unsigned polls = 0;; ++polls) {
+            bool ok = has_tag(vm, p.tag);
+#pragma unroll
+            for (int i = 0; i < kRound; ++i) ok = ok && has_tag(v[i], p.tag);
+            if (__all(ok)) break;
+            if (polls == kPollCap) {
+                l = __builtin_nanf("");
+                return;
+            }
+            if (!has_tag(vm, p.tag)) vm = tag_load(pm);
+#pragma unroll
+            for (int i = 0; i < kRound; ++i)
+                if (!has_tag(v[i], p.tag)) v[i] = tag_load(po + static_cast<size_t>(s0 + 2 * i) * kHd);
+        }
+        // Consumed: zeroed for the next launch.
+        if (mine) tag_store(pm, 0.f, 0);
+#pragma unroll
+        for (int i = 0; i < kRound; ++i)
+            if (s0 + 2 * i < n) tag_store(po + static_cast<size_t>(s0 + 2 * i) * kHd, 0.f, 0);
+        const float sm = mine && lane < kRound ? value_of(vm) : -FLT_MAX;
+        const float sl_ = __shfl(value_of(vm), lane + kRound);
+        const float mn = fmaxf(m, wave_max(sm)), f = exp2_hw(m - mn);
+        const float e = mine && lane < kRound ? exp2_hw(sm - mn) : 0.f;
+        m = mn;
+        l = fmaf(l, f, wave_sum(mine && lane < kRound ? sl_ * e : 0.f));
+        o *= f;
+#pragma unroll
+        for (int i = 0; i < kRound; ++i)
+            if (s0 + 2 * i < n) o = fmaf(value_of(v[i]), __shfl(e, i), o);
     }
-    out[h * kHd + d] = acc / L;
+}
+
+// grid (nkv, splits), block 512.
+__global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* q, const uint16_t* kc, const uint16_t* vc,
+                                                                   const int* d_pos, Partials part, float* out, int max_seq) {
+    __shared__ float so[kWaves][kGroup][kHd];  // [wave][head][column]
+    __shared__ float sml[kWaves][kGroup][2];   // [wave][head] m, l
+
+    // The group's 4 queries, the lane's 8 columns of each.
+    float qr[kGroup][8];
+#pragma unroll
+    for (int h = 0; h < kGroup; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(q + (blockIdx.x * kGroup + h) * kHd + threadIdx.x % 8 * 8 + e);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) qr[h][e + i] = v[i];
+        }
+    const int ctx = *d_pos + 1;
+    const int kvh = blockIdx.x, split = blockIdx.y, splits = gridDim.y;
+    const int tiles = (ctx + kTile - 1) / kTile, used = min(splits, (tiles + kWaves - 1) / kWaves);
+    if (split >= used) return;
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
+    const int g = lane / 8, c = lane % 8;
+    // Tiles [t, end) of this wave; the last one may reach past ctx.
+    const unsigned wi = split * kWaves + w, waves = kWaves * used;
+    int t = static_cast<int>(static_cast<uint64_t>(wi) * tiles / waves);
+    const int end = static_cast<int>(static_cast<uint64_t>(wi + 1) * tiles / waves);
+
+    // A kv head's rows as a uniform base and the lane's offset from the wave's first row (32 bits: 2^24 rows of a wave).
+    const size_t first = (static_cast<size_t>(kvh) * max_seq + static_cast<size_t>(t) * kTile) * kHd;
+    const char* K = reinterpret_cast<const char*>(kc + first);
+    const char* V = reinterpret_cast<const char*>(vc + first);
+    const int t_first = t, last_row = ctx - 1 - t * kTile;
+    auto load = [&](KvTile& kv, int tile) {  // rows past ctx read the last row again
+#pragma unroll
+        for (int r = 0; r < kTileRows; ++r) {
+            const uint32_t off = min((tile - t_first) * kTile + 8 * r + g, last_row) * (kHd * 2) + c * 16;
+            kv.k[r] = load_stream(K + off);
+            kv.v[r] = load_stream(V + off);
+        }
+    };
+    Running st;
+#pragma unroll
+    for (int h = 0; h < kGroup; ++h) {
+        st.m[h] = -FLT_MAX;
+        st.l[h] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) st.o[h][e] = 0.f;
+    }
+    if (t < end) {
+        auto step = [&](const KvTile& kv, int tile) {
+            attend(kv, qr, st, tile * kTile, g, ctx);
+        };
+        KvTile A, B;
+        load(A, t);
+        for (;;) {
+            if (t + 1 >= end) {
+                step(A, t);
+                break;
+            }
+            load(B, t + 1);
+            __builtin_amdgcn_sched_barrier(0);  // the next tile's loads go out before this tile's math
+            step(A, t);
+            if (++t + 1 >= end) {
+                step(B, t);
+                break;
+            }
+            load(A, t + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            step(B, t);
+            ++t;
+        }
+    }
+
+    // The wave's 8 token phases: every phase is rescaled to the head's maximum, then summed by exchanges that halve the
+    // values a lane holds: lane bits 5 and 4 pick the head, bit 3 the half of the lane's 8 columns.
+    float M[kGroup];
+#pragma unroll
+    for (int h = 0; h < kGroup; ++h) {
+        M[h] = phase_max(st.m[h]);
+        const float f = exp2_hw(st.m[h] - M[h]);
+        st.l[h] = phase_sum(st.l[h] * f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) st.o[h][e] *= f;
+    }
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        x[e] = fold_lanes<16>(fold_lanes<32>(st.o[0][e], st.o[1][e]), fold_lanes<32>(st.o[2][e], st.o[3][e]));
+    const bool odd = lane & 8;
+    f32x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = (odd ? x[e + 4] : x[e]) + dpp<kDppRor8>(odd ? x[e] : x[e + 4]);
+    *reinterpret_cast<f32x4*>(&so[w][(lane >> 5) + 2 * ((lane >> 4) & 1)][c * 8 + (odd ? 4 : 0)]) = y;
+    if (lane < kGroup) {
+        float m = M[0], l = st.l[0];
+#pragma unroll
+        for (int h = 1; h < kGroup; ++h)
+            if (lane == h) m = M[h], l = st.l[h];
+        sml[w][lane][0] = m;
+        sml[w][lane][1] = l;
+    }
+    __syncthreads();
+
+    // Waves 0-3 take a head each: the 8 waves' partials in wave order.
+    const int h = kvh * kGroup + w % kGroup;
+    float m = -FLT_MAX, l = 0.f, o = 0.f;
+    if (w < kGroup) {
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) m = fmaxf(m, sml[i][w][0]);
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) {
+            const float f = exp2_hw(sml[i][w][0] - m);
+            l = fmaf(sml[i][w][1], f, l);
+            o = fmaf(so[i][w][lane], f, o);
+        }
+        if (used == 1) {
+            out[h * kHd + lane] = o / l;
+        } else if (split + 1 < used) {
+            const size_t slot = static_cast<size_t>(h) * splits + split;
+            tag_store(part.o + slot * kHd + lane, o, part.tag);
+            if (lane < 2) tag_store(part.ml + slot * 2 + lane, lane ? l : m, part.tag);
+        }
+    }
+    if (split + 1 < used || used == 1) return;
+
+    // The last split: each head's other splits in two halves (waves w and w + 4), then the head's three partials.
+    float om, ol, oo;
+    merge_half(part, h, splits, used - 1, w / kGroup, lane, om, ol, oo);
+    __syncthreads();  // waves 0-3 have read so and sml
+    so[w][0][lane] = oo;
+    if (lane == 0) sml[w][0][0] = om, sml[w][0][1] = ol;
+    __syncthreads();
+    if (w < kGroup) {
+        const float m1 = sml[w + kGroup][0][0], l1 = sml[w + kGroup][0][1], o1 = so[w + kGroup][0][lane];
+        const float M = fmaxf(fmaxf(om, m1), m), f0 = exp2_hw(om - M), f1 = exp2_hw(m1 - M), f = exp2_hw(m - M);
+        out[h * kHd + lane] = (oo * f0 + o1 * f1 + o * f) / (ol * f0 + l1 * f1 + l * f);
+    }
 }
 
 // grid nh, block 256, dynamic LDS max_seq floats of scores + 16 scratch.
@@ -255,10 +481,14 @@ void launch_attention_splitk(const float* q, const uint16_t* k_cache, const uint
     CLLM_REQUIRE(hd == kHd, "attention (split-K): needs head_dim 64");
     CLLM_REQUIRE(max_seq > 0 && max_seq % kAttnChunk == 0, "attention (split-K): max_seq must be a multiple of 128");
     CLLM_REQUIRE(aligned16(q) && aligned16(k_cache) && aligned16(v_cache), "attention: pointers must be 16-byte aligned");
-    hipLaunchKernelGGL(attn_partial_kernel, dim3(nkv, max_seq / kAttnChunk), dim3(256), 0, s, q, k_cache, v_cache,
-                       d_pos, part_o, part_ml, max_seq);
-    CLLM_HIP(hipGetLastError());
-    hipLaunchKernelGGL(attn_combine_kernel, dim3(nh), dim3(kHd), 0, s, part_o, part_ml, d_pos, out, max_seq);
+    // A word takes two of the caller's floats (and the first may lie one float further on, at 8 bytes).
+    const bool slack = (reinterpret_cast<uintptr_t>(part_o) | reinterpret_cast<uintptr_t>(part_ml)) & 7;
+    const int splits = std::max(1, std::min({(max_seq / kAttnChunk - slack) / 2, kSplitBlocks / nkv, kMaxSplits}));
+    auto words = [](float* p) { return reinterpret_cast<uint64_t*>((reinterpret_cast<uintptr_t>(p) + 7) & ~uintptr_t{7}); };
+    static std::atomic<uint32_t> launches{0};
+    const Partials part{words(part_o), words(part_ml), 0xFFC00000u | (launches.fetch_add(1, std::memory_order_relaxed) & 0x3FFFFFu)};
+    hipLaunchKernelGGL(attn_split_kernel, dim3(nkv, splits), dim3(kWaves * kWave), 0, s, q, k_cache, v_cache, d_pos, part, out,
+                       max_seq);
     CLLM_HIP(hipGetLastError());
 }
 

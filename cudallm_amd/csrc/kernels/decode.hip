@@ -1144,8 +1144,6 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i) {
     i = bi;
 }
 
-constexpr int kDppRor8 = 0x128;  // row_ror:8: lane i reads lane (i + 8) mod 16 of its 16-lane row
-
 // LSE merge for contexts past 64 splits (more than 8192 positions): one wave per head, the splits in blocks of 64
 // (lane s holds split sb + s).  Pass 1 takes the maximum over every block; pass 2 adds up l e^(m - M) per block
 // and the o values in split order.  Kept out of line: it is off the hot path, and inlined its state would

@@ -37,6 +37,7 @@ constexpr int kDppXor1 = 0xB1;        // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141;  // lane i <-> 7-i inside each 8
 constexpr int kDppMirror = 0x140;      // lane i <-> 15-i inside each 16
+constexpr int kDppRor8 = 0x128;        // row_ror:8: lane i reads lane i ^ 8 inside each 16
 
 // Sum over all 64 lanes; every lane gets the same result.  Fixed association order, so the
 // result is deterministic: (((row0 + row1) + row2) + row3) of the 16-lane butterfly sums.
@@ -79,6 +80,33 @@ __device__ __forceinline__ float sum_lanes_xor(float x) {
         asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
     }
     return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+
+// The permlane swap itself on two values: afterwards a + b is, in lanes with bit M clear, a's sum over the pair
+// (l, l ^ M) and, in lanes with it set, b's sum (each pair of values is folded into one, with no selects).
+template <int M>
+__device__ __forceinline__ float fold_lanes(float x, float y) {
+    static_assert(M == 16 || M == 32, "row swaps");
+    unsigned a = __builtin_bit_cast(unsigned, x), b = __builtin_bit_cast(unsigned, y);
+    if constexpr (M == 16) {
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    } else {
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    }
+    return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+
+// max of x over lanes l and l ^ M, for M = 16 or 32.
+template <int M>
+__device__ __forceinline__ float max_lanes_xor(float x) {
+    static_assert(M == 16 || M == 32, "row swaps");
+    unsigned a = __builtin_bit_cast(unsigned, x), b = a;
+    if constexpr (M == 16) {
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    } else {
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    }
+    return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
 }
 
 // x of lane l ^ M (M a power of two below 64): quad permutes for 1 and 2, a rotation by 8 inside each 16-lane row

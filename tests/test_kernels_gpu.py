@@ -212,6 +212,92 @@ def test_attention_large_scores_are_stable():
     assert np.allclose(out, K.attention(q, k, v, 1000, NH, NKV, HD), rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("nkv,max_seq", [(8, 4096), (1, 640), (2, 128), (64, 1024), (300, 512)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_attention_launch_splits(nkv, max_seq, shift):
+    """The device-pointer launch where its division of the tokens changes: one tile or split more or less, contexts
+    that leave waves without tokens, more kv heads than workgroups; scratch whose words start off 8-byte alignment.
+    One tolerance: the 64-bit result within 2^-24 of each of the 64 products, the weight and the sums over splits,
+    about 1e-5 relative to the largest |v|."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(nkv + max_seq)
+    nh, slots = 4 * nkv, 4 * nkv * (max_seq // 128)
+    q = torch.randn(nh * 64, generator=g, device="cuda")
+    k, v = (torch.randn(nkv, max_seq, 64, generator=g, device="cuda").half() for _ in range(2))
+    part_o = torch.full((slots * 64 + 1,), 7.0, device="cuda")[shift:]
+    part_ml = torch.full((slots * 2 + 1,), 7.0, device="cuda")[shift:]
+    out = torch.empty(nh * 64, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    for ctx in (1, 2, 31, 32, 33, 100, 255, 256, 257, 288, 289, 511, 513, 640, 1000, 2049, 3969, 4095, 4096):
+        if ctx > max_seq:
+            continue
+        pos = torch.tensor([ctx - 1], dtype=torch.int32, device="cuda")
+        E.launch_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), pos.data_ptr(), part_o.data_ptr(), part_ml.data_ptr(),
+                           out.data_ptr(), nh, nkv, 64, max_seq, stream)
+        s = torch.matmul(q.double().view(nkv, 4, 64).cpu(), k[:, :ctx].double().cpu().transpose(1, 2)) * 0.125
+        ref = torch.matmul(torch.softmax(s, dim=-1), v[:, :ctx].double().cpu()).view(-1)
+        err = (out.double().cpu() - ref).abs().max().item()
+        assert err <= 1e-5 * v.abs().max().item(), f"ctx {ctx}: {err}"
+
+
+def test_attention_replayed_launch():
+    """A captured launch replayed over changing contexts (its split words are its own each time), against eager calls."""
+    import torch
+    nkv, max_seq = 8, 4096
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    q = torch.randn(nkv * 256, generator=g, device="cuda")
+    k, v = (torch.randn(nkv, max_seq, 64, generator=g, device="cuda").half() for _ in range(2))
+    pos = torch.zeros(1, dtype=torch.int32, device="cuda")
+    out, want = (torch.empty(nkv * 256, device="cuda") for _ in range(2))
+
+    def launch(dst):
+        E.launch_attention_static(q.data_ptr(), k.data_ptr(), v.data_ptr(), pos.data_ptr(), dst.data_ptr(), 4 * nkv, nkv, 64,
+                                  max_seq, torch.cuda.current_stream().cuda_stream)
+
+    launch(want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        launch(out)
+    for i, ctx in enumerate((4096, 3000, 4096, 1, 257, 4000, 256, 513)):
+        pos.fill_(ctx - 1)
+        q.mul_(-1.01)  # the words of the replay before would give another result
+        graph.replay()
+        if i % 2:
+            torch.cuda.synchronize()
+        launch(want)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), f"ctx {ctx}"
+
+
+@pytest.mark.parametrize("where", ["k", "v", "q"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_attention_non_finite(where, value):
+    """One infinity or NaN in the inputs: the outputs are the closed form's, term by term (a score of -inf weighs 0)."""
+    import torch
+    nkv, max_seq, ctx, t, d = 2, 1024, 700, 333, 5
+    g = torch.Generator(device="cuda")
+    g.manual_seed(11)
+    q = torch.rand(nkv * 256, generator=g, device="cuda") + 0.5
+    k, v = (torch.randn(nkv, max_seq, 64, generator=g, device="cuda").half() for _ in range(2))
+    k[:, ctx:] = float("nan")  # past the context: never read
+    v[:, ctx:] = float("inf")
+    if where == "q":
+        q[d] = value
+    else:
+        (k if where == "k" else v)[0, t, d] = value
+    pos = torch.tensor([ctx - 1], dtype=torch.int32, device="cuda")
+    out = torch.empty(nkv * 256, device="cuda")
+    E.launch_attention_static(q.data_ptr(), k.data_ptr(), v.data_ptr(), pos.data_ptr(), out.data_ptr(), 4 * nkv, nkv, 64,
+                              max_seq, torch.cuda.current_stream().cuda_stream)
+    s = torch.matmul(q.double().view(nkv, 4, 64).cpu(), k[:, :ctx].double().cpu().transpose(1, 2)) * 0.125
+    p = torch.exp(s - s.amax(-1, keepdim=True))
+    ref = (torch.matmul(p, v[:, :ctx].double().cpu()) / p.sum(-1, keepdim=True)).view(-1)
+    np.testing.assert_allclose(out.double().cpu().numpy(), ref.numpy(), rtol=1e-5, atol=1e-5)
+
+
 def test_silu_mul():
     gu = (np.random.default_rng(14).standard_normal(2 * 8192) * 2).astype(np.float32)
     assert np.allclose(E.kernel_silu_mul(gu), K.silu_mul(gu), rtol=1e-5)
