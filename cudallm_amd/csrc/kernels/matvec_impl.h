@@ -29,7 +29,7 @@
 //    many as can be resident)), but with KS = 1 at least enough workgroups that none takes more than
 //    64 / R passes.
 //
-// Widths with cols % 2048 != 0 or cols/2048 not in {1,4} use matvec_generic, which stages x in LDS.
+// Widths other than 2048 and 8192 use matvec_wide, which stages x in LDS.
 #pragma once
 
 #include <algorithm>
@@ -357,73 +357,278 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     }
 }
 
-// Any cols that is a multiple of 1024 (up to 12288): x^ staged in LDS, one wave per row.
-template <WType WT, Epilogue EP, bool NORM>
-__global__ void __launch_bounds__(kThreads) matvec_generic(MatvecArgs a) {
+// ---- any width: cols a multiple of 1024, up to 12288 -----------------------------------------------------
+//
+// Bound by the weight bytes (int4 by instruction issue beside them).  x^ is staged in LDS once per workgroup in the order
+// in which the lanes of a wave read it, so a wave takes whole rows of any width: a step is one 1 KiB line (64 chunks) of
+// two rows, the gate and the up row with SWIGLU, else two neighbours, which share the LDS reads of x^.  The quantised
+// types stage x^ as the digit words of digits.h (a line's digit d of lane l at [line][d][l], 16 bytes; a third to a half
+// of the instructions of converting every weight), bf16 as float4s ([line][quad][l]).  The steps of all of a wave's rows
+// are one sequence with kDepth steps in flight; the loads are buffer loads, so the ones past the wave's last row and past
+// a row's end (widths that are not a whole number of lines) return 0 without a memory access and no load sits under a
+// branch.  Row sums wait in LDS for the wave's end, so no store sits in the loop either.
+constexpr int kWideWaves = 8, kWideThreads = kWideWaves * kWave;
+constexpr int kWideMaxUnits = 64;  // row pairs per wave
+constexpr int kXPairs = 12288 / 8 / kWideThreads;  // a thread stages 8 columns at a time
+// Steps in flight per wave.  int4 has the most instructions per step, and a third copy of them in the loop costs more
+// than it hides: 24576 x 4096 with depths 2, 3 and 4: bf16 35.9 / 34.9 / 34.9 us, int8 21.0 / 19.2 / 19.3, int4 12.3 /
+// 13.2 / 14.2; 1000 x 1024: bf16 3.1 / 3.1 / 3.5, int8 3.4 / 3.5 / 3.9, int4 3.6 / 4.0 / 4.2.
+template <WType WT>
+constexpr int kDepth = WT == WType::INT4 ? 2 : 3;
+
+// The fixed-point scale here fills the digits' whole range (|xi| up to about 2^23, a bit more than digits.h's own words
+// hold), so that the rounding of x^ adds no more than the sums in 32 bits did: 24576 x 4096 int4 with SWIGLU, against 64
+// bits: 5.1e-7 converting every weight, 8.1e-7 with |xi| < 2^22.
+template <WType WT>
+__device__ __forceinline__ int wide_exponent(float m) {
+    if (!(m > 0.f) || !(m < INFINITY)) return 0;
+    constexpr float kMost = WT == WType::INT8 ? 8355700.f : 7829350.f;  // 127 (1 + 256 + 256^2), 7 (1 + 16 + ... + 16^5)
+    const int e = min(22 - ilogbf(m), 126);
+    return ldexpf(m, e) > kMost ? e - 1 : e;
+}
+__device__ __forceinline__ uint32_t wide_word(float v, float scale, uint32_t C) {
+    return static_cast<uint32_t>(static_cast<int>(rintf(v * scale))) + C;
+}
+
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+__device__ __forceinline__ Rsrc make_rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+constexpr int kAuxNt = 2;  // non-temporal
+
+template <WType WT>
+struct Wide {
     using F = Fmt<WT>;
-    extern __shared__ float xs[];
-    __shared__ float scratch[16];
-    constexpr bool GLU = EP == Epilogue::SWIGLU;
-    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-    const int out_rows = GLU ? a.rows / 2 : a.rows;
-    float inv = 1.f;
-    if constexpr (NORM) {
-        float ss = 0.f;
-        for (int j = tid; j < a.cols; j += kThreads) ss += a.x[j] * a.x[j];
-        ss = block_sum(ss, scratch);
-        inv = rsqrtf(ss / static_cast<float>(a.cols) + a.eps);
+    static constexpr int Q = WT == WType::INT4 ? 6 : WT == WType::INT8 ? 3 : 2;  // 16-byte words of x^ per chunk
+    static __host__ __device__ int lines(int cols) { return (cols / F::CPC + kWave - 1) / kWave; }
+    // x^, then the row sums.
+    static size_t smem(int cols, int units_per_wave) {
+        return static_cast<size_t>(lines(cols)) * kWave * Q * 16 + sizeof(float) * kWideWaves * 2 * units_per_wave;
     }
-    for (int j = tid; j < a.cols; j += kThreads) xs[j] = NORM ? a.x[j] * inv * a.norm_w[j] : a.x[j];
+};
+
+template <WType WT, Epilogue EP, bool NORM>
+__global__ void __launch_bounds__(kWideThreads) matvec_wide(MatvecArgs a, int units, int max_units) {
+    using F = Fmt<WT>;
+    constexpr bool GLU = EP == Epilogue::SWIGLU, DIG = WT != WType::BF16;
+    constexpr int Q = Wide<WT>::Q;
+    extern __shared__ u32x4 xs[];  // [line][Q][lane]
+    __shared__ float sred[kWideWaves], mred[kWideWaves];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
+    const int nchunk = a.cols / F::CPC, nk = Wide<WT>::lines(a.cols), rem = nchunk - (nk - 1) * kWave;
+    float* const sums = reinterpret_cast<float*>(xs + nk * Q * kWave) + wave * 2 * max_units;
+
+    // Units [u0, u0 + n) of this wave.
+    const int64_t wi = blockIdx.x * kWideWaves + wave, nw = gridDim.x * kWideWaves;
+    const int u0 = static_cast<int>(wi * units / nw), n = static_cast<int>((wi + 1) * units / nw) - u0;
+    const int out_rows = GLU ? a.rows / 2 : a.rows;
+
+    // x first, so that its wait does not include the weights.
+    f32x4 xv[kXPairs][2], nv[NORM ? kXPairs : 1][2];
+    const int pairs = a.cols / 8;  // a multiple of 128: all of a wave's lanes hold one, or none
+#pragma unroll
+    for (int i = 0; i < kXPairs; ++i) {
+        xv[i][0] = xv[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (NORM) nv[i][0] = nv[i][1] = xv[i][0];
+        if (i * kWideThreads + wave * kWave < pairs) {
+            const int j = 2 * (i * kWideThreads + tid);
+            xv[i][0] = reinterpret_cast<const f32x4*>(a.x)[j];
+            xv[i][1] = reinterpret_cast<const f32x4*>(a.x)[j + 1];
+            if constexpr (NORM) {
+                nv[i][0] = reinterpret_cast<const f32x4*>(a.norm_w)[j];
+                nv[i][1] = reinterpret_cast<const f32x4*>(a.norm_w)[j + 1];
+            }
+        }
+    }
+
+    // The wave's rows as two buffers: rows r0, r0 + pitch, ... and their partners.
+    const uint32_t rb = static_cast<uint32_t>(row_bytes<WT>(a.cols)), pitch = GLU ? rb : 2 * rb;
+    const int r0 = GLU ? u0 : 2 * u0;
+    const char* w0 = static_cast<const char*>(a.w) + static_cast<size_t>(r0) * rb;
+    const int rows_here = GLU ? n : min(2 * n, a.rows - r0);
+    const Rsrc wa = make_rsrc(w0, rows_here * rb);
+    const Rsrc wb = GLU ? make_rsrc(w0 + static_cast<size_t>(out_rows) * rb, rows_here * rb) : wa;
+    const uint32_t second = GLU ? 0 : rb;
+    // int4 group scales: one fp16 per 128 columns (4 chunks).
+    const uint32_t sb = a.cols / 128 * 2, spitch = GLU ? sb : 2 * sb, ssecond = GLU ? 0 : sb;
+    const char* s0 = static_cast<const char*>(a.scales) + static_cast<size_t>(r0) * sb;
+    const Rsrc sa = WT == WType::INT4 ? make_rsrc(s0, rows_here * sb) : wa;
+    const Rsrc sbu = WT == WType::INT4 && GLU ? make_rsrc(s0 + static_cast<size_t>(out_rows) * sb, rows_here * sb) : sa;
+
+    struct Step {
+        u32x4 v[2];
+        uint16_t g[2];
+    };
+    const uint32_t full_off = lane * 16, last_off = lane < rem ? full_off : 0x80000000u;
+    const uint32_t full_soff = lane / 4 * 2, last_soff = lane < rem ? full_soff : 0x80000000u;
+    uint32_t row_off = 0, row_soff = 0;
+    int lk = 0;  // the next step's line
+    auto load = [&](Step& b) {
+        const bool last = lk == nk - 1;
+        const uint32_t off = row_off + lk * 1024 + (last ? last_off : full_off);
+        b.v[0] = __builtin_amdgcn_raw_buffer_load_b128(wa, off, 0, kAuxNt);
+        b.v[1] = __builtin_amdgcn_raw_buffer_load_b128(wb, off + second, 0, kAuxNt);
+        if constexpr (WT == WType::INT4) {
+            const uint32_t so = row_soff + lk * 32 + (last ? last_soff : full_soff);
+            b.g[0] = __builtin_amdgcn_raw_buffer_load_b16(sa, so, 0, 0);
+            b.g[1] = __builtin_amdgcn_raw_buffer_load_b16(sbu, so + ssecond, 0, 0);
+        }
+        row_off += last ? pitch : 0;
+        row_soff += last ? spitch : 0;
+        lk = last ? 0 : lk + 1;
+    };
+    Step st[kDepth<WT>];
+#pragma unroll
+    for (int d = 0; d < kDepth<WT>; ++d) load(st[d]);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // The sum of squares (norm) and the largest |x norm_w| (digits; infinite if any input is infinite or NaN).
+    [[maybe_unused]] float inv = 1.f, dsc = 1.f, scale = 1.f;
+    if constexpr (NORM || DIG) {
+        float ss = 0.f, mx = 0.f;
+#pragma unroll
+        for (int i = 0; i < kXPairs; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float v = xv[i][e / 4][e % 4];
+                ss = fmaf(v, v, ss);
+                if constexpr (DIG) {
+                    const float t = NORM ? v * nv[i][e / 4][e % 4] : v;
+                    mx = fabsf(t) < INFINITY ? fmaxf(mx, fabsf(t)) : INFINITY;
+                }
+            }
+        if constexpr (NORM) ss = wave_sum(ss);
+        if constexpr (DIG) mx = wave_max(mx);
+        if (lane == 0) sred[wave] = ss, mred[wave] = mx;
+        __syncthreads();
+        ss = 0.f, mx = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWideWaves; ++w) ss += sred[w], mx = fmaxf(mx, mred[w]);
+        if constexpr (NORM) inv = rsqrtf(ss / static_cast<float>(a.cols) + a.eps);
+        if constexpr (DIG) {
+            const int e = wide_exponent<WT>(mx * inv);
+            scale = ldexpf(1.f, e);
+            dsc = mx * inv < INFINITY ? ldexpf(1.f, -e) : __builtin_nanf("");
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kXPairs; ++i) {
+        // A whole number of lines: columns past the row's end stay 0.
+        if (i * kWideThreads + wave * kWave >= nk * kWave * F::CPC / 8) continue;
+        const int j = i * kWideThreads + tid;  // columns 8 j .. 8 j + 7
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            v[e] = xv[i][e / 4][e % 4];
+            if constexpr (NORM) v[e] = v[e] * inv * nv[i][e / 4][e % 4];
+        }
+        uint32_t* const xw = reinterpret_cast<uint32_t*>(xs);
+        if constexpr (WT == WType::BF16) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                xs[(j / kWave * Q + q) * kWave + j % kWave] =
+                    __builtin_bit_cast(u32x4, f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]});
+        } else if constexpr (WT == WType::INT8) {
+            const int c = j / 2, at = (c / kWave * Q * kWave + c % kWave) * 4 + j % 2 * 2;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                uint32_t P[3];
+                byte_planes(wide_word(v[4 * h], scale, 0x808080u), wide_word(v[4 * h + 1], scale, 0x808080u),
+                            wide_word(v[4 * h + 2], scale, 0x808080u), wide_word(v[4 * h + 3], scale, 0x808080u), P);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) xw[at + d * kWave * 4 + h] = P[d] ^ 0x80808080u;
+            }
+        } else {
+            const int c = j / 4, at = (c / kWave * Q * kWave + c % kWave) * 4 + j % 4;
+            uint32_t u[8], w[6];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) u[e] = wide_word(v[e], scale, 0x888888u);
+            nibble_words(u, w);
+#pragma unroll
+            for (int d = 0; d < 6; ++d) xw[at + d * kWave * 4] = w[d] ^ 0x88888888u;
+        }
+    }
     __syncthreads();
 
-    const size_t rb = row_bytes<WT>(a.cols);
-    const int nchunk = a.cols / F::CPC;
-    const int groups_per_row = a.cols / 128;
-    for (int r = blockIdx.x * 4 + wave; r < out_rows; r += gridDim.x * 4) {
-        float s = 0.f, su = 0.f;
-        for (int c = lane; c < nchunk; c += kWave) {
-            const float* x = xs + c * F::CPC;
-            const char* p = static_cast<const char*>(a.w) + static_cast<size_t>(r) * rb + c * 16;
-            float t = chunk_dot<WT>(load_stream(p), x);
-            float tu = GLU ? chunk_dot<WT>(load_stream(p + static_cast<size_t>(out_rows) * rb), x) : 0.f;
-            if constexpr (WT != WType::BF16) {
-                float xsum = 0.f;
+    // Row sums: float for bf16 and int4 (per line, times the group scale), exact integers per digit for int8.
+    float acc[2] = {0.f, 0.f};
+    [[maybe_unused]] int ia[2][3] = {{0, 0, 0}, {0, 0, 0}};
+    int k = 0, u = 0;
+    auto step = [&](const Step& b) {
+        u32x4 x[Q];
 #pragma unroll
-                for (int j = 0; j < F::CPC; ++j) xsum += x[j];
-                t -= kBias<WT> * xsum;
-                if constexpr (GLU) tu -= kBias<WT> * xsum;
+        for (int q = 0; q < Q; ++q) x[q] = xs[(k * Q + q) * kWave + lane];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if constexpr (WT == WType::BF16) {
+                float xf[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) xf[e] = __builtin_bit_cast(f32x4, x[e / 4])[e % 4];
+                acc[i] += chunk_dot<WT>(b.v[i], xf);
+            } else if constexpr (WT == WType::INT8) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d)
+                        ia[i][d] = __builtin_amdgcn_sdot4(static_cast<int>(b.v[i][t]), static_cast<int>(x[d][t]), ia[i][d], false);
+            } else {
+                int c[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int w = static_cast<int>(b.v[i][t] ^ 0x88888888u);
+#pragma unroll
+                    for (int d = 0; d < 6; ++d) c[d] = __builtin_amdgcn_sdot8(w, static_cast<int>(x[d][t]), c[d], false);
+                }
+                const int p0 = c[0] + 16 * c[1], p1 = c[2] + 16 * c[3], p2 = c[4] + 16 * c[5];
+                acc[i] = fmaf(fmaf(static_cast<float>(p2), 65536.f, static_cast<float>(p0 + 256 * p1)), half_bits_to_float(b.g[i]), acc[i]);
             }
-            if constexpr (WT == WType::INT4) {
-                const uint16_t* sc = static_cast<const uint16_t*>(a.scales);
-                const int gi = c * F::CPC / 128;
-                t *= half_bits_to_float(sc[static_cast<size_t>(r) * groups_per_row + gi]);
-                if constexpr (GLU) tu *= half_bits_to_float(sc[static_cast<size_t>(r + out_rows) * groups_per_row + gi]);
-            }
-            s += t;
-            su += tu;
         }
-        s = wave_sum(s);
-        su = GLU ? wave_sum(su) : 0.f;
-        if (lane == 0) {
-            if constexpr (WT == WType::INT8) {
-                const float* sc = static_cast<const float*>(a.scales);
-                s *= sc[r];
-                if constexpr (GLU) su *= sc[r + out_rows];
-            }
-            store_out<EP>(a.y, r, s, su);
+        if (++k == nk) {
+            if constexpr (WT == WType::INT8)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    acc[i] = fmaf(fmaf(static_cast<float>(ia[i][2]), 256.f, static_cast<float>(ia[i][1])), 256.f, static_cast<float>(ia[i][0]));
+                    ia[i][0] = ia[i][1] = ia[i][2] = 0;
+                }
+            const float t = rows_sum<2>(acc, lane);
+            if (lane < 2) sums[2 * u + lane] = t;
+            acc[0] = acc[1] = 0.f;
+            k = 0;
+            ++u;
         }
+    };
+    for (int s = n * nk; s > 0; s -= kDepth<WT>) {
+#pragma unroll
+        for (int d = 0; d < kDepth<WT>; ++d) {
+            if (d == 0 || s > d) step(st[d]);
+            load(st[d]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int i = lane; i < (GLU ? n : 2 * n); i += kWave) {
+        const int r = r0 + i;
+        if (r >= out_rows) break;
+        float d = sums[GLU ? 2 * i : i] * dsc, du = GLU ? sums[2 * i + 1] * dsc : 0.f;
+        if constexpr (WT == WType::INT8) {
+            const float* sc = static_cast<const float*>(a.scales);
+            d *= sc[r];
+            if constexpr (GLU) du *= sc[r + out_rows];
+        }
+        store_out<EP>(a.y, r, d, du);
     }
 }
 
 // Launches a matvec kernel; when the thread has armed kernel events (arm_kernel_events), the dispatch itself
 // records them at the kernel's start and end, so a benchmark times the kernel without the launch gap.
-template <typename K>
-void dispatch(K kernel, int grid, size_t smem, hipStream_t s, const MatvecArgs& a) {
+template <typename K, typename... Args>
+void dispatch(K kernel, int grid, int threads, size_t smem, hipStream_t s, const Args&... args) {
     KernelEvents ev = take_kernel_events();
     if (ev.start)
-        hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), static_cast<uint32_t>(smem), s, ev.start, ev.stop, 0u, a);
+        hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(threads), static_cast<uint32_t>(smem), s, ev.start, ev.stop, 0u, args...);
     else
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), smem, s, a);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), smem, s, args...);
     CLLM_HIP(hipGetLastError());
 }
 
@@ -447,17 +652,18 @@ void launch_fast(const MatvecArgs& a, hipStream_t s) {
     const int per_cu = grid_per_cu(WT, EP, a.rows, a.cols);
     const int grid = std::max(std::min(need, device_cu_count() * (per_cu > 0 ? per_cu : occ)),
                               KS == 1 ? (need + kMaxPasses<R> - 1) / kMaxPasses<R> : 0);
-    dispatch(k, grid, 0, s, a);
+    dispatch(k, grid, kThreads, 0, s, a);
 }
 
 template <WType WT, Epilogue EP, bool NORM>
-void launch_generic(const MatvecArgs& a, hipStream_t s) {
-    auto k = matvec_generic<WT, EP, NORM>;
-    const size_t smem = static_cast<size_t>(a.cols) * sizeof(float);
-    const int occ = resident_blocks(k, smem);
-    const int out_rows = EP == Epilogue::SWIGLU ? a.rows / 2 : a.rows;
-    const int grid = std::min((out_rows + 3) / 4, device_cu_count() * occ);
-    dispatch(k, grid, smem, s, a);
+void launch_wide(const MatvecArgs& a, hipStream_t s) {
+    const int units = EP == Epilogue::SWIGLU ? a.rows / 2 : (a.rows + 1) / 2;
+    // Two workgroups per CU, fewer if that leaves the waves with the same number of units, more so that none has over
+    // kWideMaxUnits.
+    const int most = device_cu_count() * 2 * kWideWaves;
+    const int per_wave = std::min((units + most - 1) / most, kWideMaxUnits);
+    const int grid = (units + kWideWaves * per_wave - 1) / (kWideWaves * per_wave);
+    dispatch(matvec_wide<WT, EP, NORM>, grid, kWideThreads, Wide<WT>::smem(a.cols, per_wave), s, a, units, per_wave);
 }
 
 template <WType WT, Epilogue EP, bool NORM, int KS>
@@ -475,7 +681,7 @@ template <WType WT, Epilogue EP, bool NORM>
 void pick_shape(int rpb, const MatvecArgs& a, hipStream_t s) {
     if (a.cols == 2048) return pick_r<WT, EP, NORM, 1>(rpb, a, s);
     if (a.cols == 8192) return pick_r<WT, EP, NORM, 4>(rpb, a, s);
-    return launch_generic<WT, EP, NORM>(a, s);
+    return launch_wide<WT, EP, NORM>(a, s);
 }
 
 template <WType WT>

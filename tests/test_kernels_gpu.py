@@ -100,6 +100,66 @@ def test_matvec_generic_and_ragged(wtype, rows, cols, epilogue):
     _check_matvec(wtype, epilogue, 1, 4, rows, cols, seed=rows + 3 * cols)
 
 
+@pytest.mark.parametrize("wtype", ["bf16", "int8", "int4"])
+@pytest.mark.parametrize("rows,cols,epilogue", [(1, 1024, "store"), (3, 5120, "add"), (2, 11264, "swiglu"),
+                                                (8191, 1024, "store"), (8194, 7168, "swiglu"), (600000, 1024, "store")])
+def test_matvec_wide_rows(wtype, rows, cols, epilogue):
+    """The any-width kernel where its division of the rows changes: one row, an odd last row, widths that end inside a
+    line, waves without rows, waves with as many rows as they take (600000 rows).  The error against 64 bits stays
+    under cols roundings of 2^-24 of the inputs, in the root mean square about sqrt(cols) of them: 1e-5 is ten times."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows + cols)
+    n = rows // 2 if epilogue == "swiglu" else rows
+    q = torch.randint(-8 if wtype == "int4" else -127, 8 if wtype == "int4" else 128, (rows, cols), generator=g,
+                      device="cuda", dtype=torch.int8)
+    scales = None
+    if wtype == "bf16":
+        w = q.to(torch.bfloat16)
+    elif wtype == "int8":
+        w, scales = q, torch.rand(rows, generator=g, device="cuda") + 0.5
+    else:
+        u = (q + 8).view(rows, cols // 2, 2).to(torch.uint8)
+        w, scales = u[..., 0] | (u[..., 1] << 4), (torch.rand(rows, cols // 128, generator=g, device="cuda") + 0.5).half()
+    x, norm = torch.randn(cols, generator=g, device="cuda"), torch.rand(cols, generator=g, device="cuda") + 0.5
+    y0 = torch.randn(n, generator=g, device="cuda")
+    y = torch.cat([y0, torch.full((8,), 3.0, device="cuda")])
+    E.launch_matvec(wtype, epilogue, 0, w.data_ptr(), None if scales is None else scales.data_ptr(), x.data_ptr(),
+                    norm.data_ptr(), 1e-5, y.data_ptr(), rows, cols, torch.cuda.current_stream().cuda_stream)
+    xn = x.double()
+    xn = xn * torch.rsqrt((xn * xn).mean() + 1e-5) * norm.double()
+    d = torch.empty(rows, dtype=torch.float64, device="cuda")
+    for r in range(0, rows, 50000):
+        m = q[r:r + 50000].double()
+        if wtype == "int8":
+            m *= scales[r:r + 50000, None].double()
+        elif wtype == "int4":
+            m = (m.view(len(m), -1, 128) * scales[r:r + 50000, :, None].double()).view(len(m), cols)
+        d[r:r + 50000] = m @ xn
+    ref = torch.nn.functional.silu(d[:n]) * d[n:] if epilogue == "swiglu" else d + y0.double() if epilogue == "add" else d
+    assert (y[:n].double() - ref).norm() <= 1e-5 * ref.norm()
+    assert bool((y[n:] == 3.0).all())  # nothing past the outputs
+
+
+@pytest.mark.parametrize("wtype", ["bf16", "int8", "int4"])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_matvec_wide_non_finite_input(wtype, norm, value):
+    """An infinite or NaN input does not come out as a number: with a norm, and for the quantised types, every output is
+    NaN; plain bf16 outputs are the infinity with the weight's sign."""
+    import torch
+    rows, cols = 40, 3072
+    w, s, w64 = _operands(wtype, rows, cols, 5)
+    x = np.random.default_rng(6).standard_normal(cols).astype(np.float32)
+    x[1000] = value
+    y = E.kernel_matvec("opt", wtype, "store", int(norm), 0, w, s, x, np.ones(cols, np.float32), 1e-5, None, rows, cols)
+    if wtype == "bf16" and not norm:
+        want = w64[:, 1000] * value
+        np.testing.assert_array_equal(y, want.astype(np.float32))
+    else:
+        assert np.isnan(y).all()
+
+
 def test_stream_read_timed_hook():
     """The bandwidth kernel on a device buffer through its timed hook: every launch shape records both events, and the
     sink (written only for one XOR-folded word that a zero buffer never gives) stays untouched."""
