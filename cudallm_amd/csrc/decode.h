@@ -44,7 +44,8 @@ struct DecodeParams {
     uint64_t* tact;  // [n_layers][inter]       SwiGLU output
     uint64_t* targ;  // [grid][2]               per-workgroup argmax (value, index)
     float* logits;
-    int* d_token;
+    int* d_token;  // the last argmax; this step's input when `token` is negative
+    int token;     // this step's input token, or -1
     int* d_pos;
     unsigned* d_step;  // launch counter: epoch base of the tags, never reset
     unsigned* d_err;   // sticky: set when a wait exceeded its bound

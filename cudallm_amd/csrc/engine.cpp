@@ -69,6 +69,10 @@ private:
     size_t size_ = 0;
 };
 
+// The results block a step leaves for the host: the token, the persistent kernel's error flag (a line of its own), then
+// the logits.
+constexpr size_t kErrorAt = 128, kLogitsAt = 256;
+
 // Records everything `record` enqueues on `s` into an executable graph.  The capture is ended on every
 // path, so a failure inside `record` never leaves the stream capturing.
 void capture_graph(hipStream_t s, const std::function<void()>& record, hipGraph_t* graph, hipGraphExec_t* exec) {
@@ -136,10 +140,10 @@ Engine::Engine(const std::string& path, const EngineOptions& opts) : opts_(opts)
         ArenaPlan ap;
         const size_t at_x = ap.reserve<float>(H), at_xb = ap.reserve<float>(H), at_qkv = ap.reserve<float>(QKV),
                      at_att = ap.reserve<float>(NH * D), at_tmp = ap.reserve<float>(H), at_gu = ap.reserve<float>(2 * I),
-                     at_act = ap.reserve<float>(I), at_logits = ap.reserve<float>(V),
+                     at_act = ap.reserve<float>(I), at_results = ap.reserve<char>(kLogitsAt + V * sizeof(float)),
                      at_po = ap.reserve<float>(NH * NS * D), at_pml = ap.reserve<float>(NH * NS * 2),
                      at_av = ap.reserve<float>(kArgmaxParts), at_ai = ap.reserve<int>(kArgmaxParts),
-                     at_tok = ap.reserve<int>(1), at_pos = ap.reserve<int>(1),
+                     at_pos = ap.reserve<int>(1),
                      at_k = ap.reserve<uint16_t>(L * KV * S * D), at_v = ap.reserve<uint16_t>(L * KV * S * D),
                      at_res = ap.reserve<float>((L + 1) * H);
         // Tagged buffers of the persistent kernel, contiguous so that one clear covers them all.
@@ -149,8 +153,7 @@ Engine::Engine(const std::string& path, const EngineOptions& opts) : opts_(opts)
                      at_tpart = ap.reserve<uint64_t>(n_part), at_tact = ap.reserve<uint64_t>(L * I),
                      at_targ = ap.reserve<uint64_t>(2 * kDecodeMaxGrid);
         const size_t at_tags_end = ap.size();
-        const size_t at_layers = ap.reserve<DecodeLayer>(L), at_step = ap.reserve<unsigned>(1),
-                     at_err = ap.reserve<unsigned>(1), at_probe = ap.reserve<unsigned>(2),
+        const size_t at_layers = ap.reserve<DecodeLayer>(L), at_step = ap.reserve<unsigned>(1), at_probe = ap.reserve<unsigned>(2),
                      at_stamps = ap.reserve<unsigned long long>(static_cast<size_t>(grid_) * kStampSlots);
         CLLM_HIP(hipMalloc(&arena_, ap.size()));
         CLLM_HIP(hipMemset(arena_, 0, ap.size()));
@@ -163,12 +166,14 @@ Engine::Engine(const std::string& path, const EngineOptions& opts) : opts_(opts)
         tmp_ = static_cast<float*>(at(at_tmp));
         gu_ = static_cast<float*>(at(at_gu));
         act_ = static_cast<float*>(at(at_act));
-        logits_ = static_cast<float*>(at(at_logits));
+        results_ = static_cast<char*>(at(at_results));
+        logits_ = reinterpret_cast<float*>(results_ + kLogitsAt);
+        d_token_ = reinterpret_cast<int*>(results_);
+        CLLM_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_results_), kLogitsAt + V * sizeof(float), hipHostMallocDefault));
         part_o_ = static_cast<float*>(at(at_po));
         part_ml_ = static_cast<float*>(at(at_pml));
         arg_v_ = static_cast<float*>(at(at_av));
         arg_i_ = static_cast<int*>(at(at_ai));
-        d_token_ = static_cast<int*>(at(at_tok));
         d_pos_ = static_cast<int*>(at(at_pos));
         k_cache_ = static_cast<uint16_t*>(at(at_k));
         v_cache_ = static_cast<uint16_t*>(at(at_v));
@@ -208,9 +213,10 @@ Engine::Engine(const std::string& path, const EngineOptions& opts) : opts_(opts)
         dp_.targ = static_cast<uint64_t*>(at(at_targ));
         dp_.logits = logits_;
         dp_.d_token = d_token_;
+        dp_.token = -1;
         dp_.d_pos = d_pos_;
         dp_.d_step = static_cast<unsigned*>(at(at_step));
-        dp_.d_err = static_cast<unsigned*>(at(at_err));
+        dp_.d_err = reinterpret_cast<unsigned*>(results_ + kErrorAt);
         dp_.eps = c.rms_eps;
         const char* stall = std::getenv("CUDALLM_STALL");  // timing perturbation, tests only
         dp_.stall = stall ? static_cast<unsigned>(std::strtoul(stall, nullptr, 0)) : 0u;
@@ -242,6 +248,8 @@ void Engine::release() noexcept {
     graph_ = nullptr;
     if (arena_) check(hipFree(arena_), "hipFree");
     arena_ = nullptr;
+    if (host_results_) check(hipHostFree(host_results_), "hipHostFree");
+    host_results_ = nullptr;
     if (stream_) check(hipStreamDestroy(stream_), "hipStreamDestroy");
     stream_ = nullptr;
 }
@@ -359,16 +367,6 @@ void Engine::launch_persistent(const DecodeParams& p) {
     ++launches_;
 }
 
-void Engine::raise_if_kernel_failed() {
-    if (!persistent_) return;
-    unsigned flag = 0;
-    CLLM_HIP(hipMemcpy(&flag, dp_.d_err, sizeof(flag), hipMemcpyDeviceToHost));
-    if (flag)
-        throw DeviceError(
-            "persistent decode kernel: a wait on another workgroup ran past its bound, so this sequence's results are "
-            "invalid; reset() starts a new sequence");
-}
-
 // ---- steps ----------------------------------------------------------------------------------
 
 void Engine::reset() {
@@ -392,12 +390,27 @@ void Engine::begin_step(const char* who, int token) {
         throw SequenceFull(std::string(who) + ": sequence full at max_seq_len positions; reset() starts a new one");
     if (token < -1 || token >= config().vocab)
         throw ArgError(std::string(who) + ": token must be -1 or a vocabulary index");
-    if (token >= 0) launch_set_token(d_token_, token, stream_);
+    // The persistent kernel takes the token as an argument; the program's embedding reads it from the device.
+    if (persistent_)
+        dp_.token = token;
+    else if (token >= 0)
+        launch_set_token(d_token_, token, stream_);
 }
 
-void Engine::read_outputs(float* logits_out, int* next_token_out) {
-    if (logits_out) CLLM_HIP(hipMemcpy(logits_out, logits_, sizeof(float) * config().vocab, hipMemcpyDeviceToHost));
-    if (next_token_out) CLLM_HIP(hipMemcpy(next_token_out, d_token_, sizeof(int), hipMemcpyDeviceToHost));
+// Waits for the step and reads what it left: one copy of the results block (up to the error flag, or with the logits) to
+// pinned memory behind the step on its stream, and one wait.
+void Engine::finish_step(float* logits_out, int* next_token_out) {
+    const size_t logit_bytes = sizeof(float) * config().vocab;
+    CLLM_HIP(hipMemcpyAsync(host_results_, results_, kLogitsAt + (logits_out ? logit_bytes : 0), hipMemcpyDeviceToHost, stream_));
+    CLLM_HIP(hipStreamSynchronize(stream_));
+    unsigned flag = 0;
+    std::memcpy(&flag, host_results_ + kErrorAt, sizeof(flag));
+    if (flag && persistent_)
+        throw DeviceError(
+            "persistent decode kernel: a wait on another workgroup ran past its bound, so this sequence's results are "
+            "invalid; reset() starts a new sequence");
+    if (logits_out) std::memcpy(logits_out, host_results_ + kLogitsAt, logit_bytes);
+    if (next_token_out) std::memcpy(next_token_out, host_results_, sizeof(int));
 }
 
 void Engine::step(int token, float* logits_out, int* next_token_out) {
@@ -414,9 +427,7 @@ void Engine::step(int token, float* logits_out, int* next_token_out) {
     }
     host_pos_ += 1;
     if (!logits_out && !next_token_out) return;  // fully asynchronous
-    CLLM_HIP(hipStreamSynchronize(stream_));
-    raise_if_kernel_failed();
-    read_outputs(logits_out, next_token_out);
+    finish_step(logits_out, next_token_out);
 }
 
 void Engine::step_debug(int token, float* residuals_out, float* logits_out, int* next_token_out) {
@@ -430,11 +441,9 @@ void Engine::step_debug(int token, float* residuals_out, float* logits_out, int*
         run_program(true);
     }
     host_pos_ += 1;
-    CLLM_HIP(hipStreamSynchronize(stream_));
-    raise_if_kernel_failed();
+    finish_step(logits_out, next_token_out);
     const ModelConfig& c = config();
     CLLM_HIP(hipMemcpy(residuals_out, d_res_, sizeof(float) * (c.n_layers + 1) * c.hidden, hipMemcpyDeviceToHost));
-    read_outputs(logits_out, next_token_out);
 }
 
 int Engine::step_profile(int token, unsigned long long* stamps_out, long capacity) {
@@ -448,8 +457,7 @@ int Engine::step_profile(int token, unsigned long long* stamps_out, long capacit
     p.stamps = d_stamps_;
     launch_persistent(p);
     host_pos_ += 1;
-    CLLM_HIP(hipStreamSynchronize(stream_));
-    raise_if_kernel_failed();
+    finish_step(nullptr, nullptr);
     CLLM_HIP(hipMemcpy(stamps_out, d_stamps_, bytes, hipMemcpyDeviceToHost));
     return grid_;
 }
@@ -464,8 +472,7 @@ void Engine::step_trace(int token, float* trace_out, long capacity, float* logit
     p.residuals = d_res_;
     launch_persistent(p);
     host_pos_ += 1;
-    CLLM_HIP(hipStreamSynchronize(stream_));
-    raise_if_kernel_failed();
+    finish_step(logits_out, next_token_out);
     CLLM_HIP(hipMemcpy(trace_out + t.residuals, d_res_, sizeof(float) * (c.n_layers + 1) * c.hidden,
                        hipMemcpyDeviceToHost));
     // Each tagged word holds its fp32 value in the low half.
@@ -481,7 +488,6 @@ void Engine::step_trace(int token, float* trace_out, long capacity, float* logit
     unpack(dp_.tatt, t.xa - t.att, trace_out + t.att);
     unpack(dp_.txa, t.act - t.xa, trace_out + t.xa);
     unpack(dp_.tact, t.total - t.act, trace_out + t.act);
-    read_outputs(logits_out, next_token_out);
 }
 
 }  // namespace cllm

@@ -68,8 +68,7 @@ private:
     // or -1 (reuse the device argmax).
     void begin_step(const char* who, int token);
     void launch_persistent(const DecodeParams& p);
-    void read_outputs(float* logits_out, int* next_token_out);
-    void raise_if_kernel_failed();
+    void finish_step(float* logits_out, int* next_token_out);
     void build_program();
     void run_program(bool debug);
     void release() noexcept;
@@ -91,6 +90,8 @@ private:
     hipGraphExec_t graph_exec_ = nullptr;
 
     void* arena_ = nullptr;  // every activation buffer, one allocation
+    char* results_ = nullptr;       // the token, the error flag and the logits, in the arena
+    char* host_results_ = nullptr;  // their pinned host copy
     float *x_ = nullptr, *xb_ = nullptr, *qkv_ = nullptr, *att_ = nullptr, *tmp_ = nullptr, *gu_ = nullptr,
           *act_ = nullptr, *logits_ = nullptr, *part_o_ = nullptr, *part_ml_ = nullptr, *arg_v_ = nullptr;
     int *arg_i_ = nullptr, *d_token_ = nullptr, *d_pos_ = nullptr;

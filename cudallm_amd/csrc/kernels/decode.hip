@@ -1317,7 +1317,7 @@ __global__ void __launch_bounds__(kThreads) decode_kernel(DecodeParams p) {
     const int G = gridDim.x, NW = G * kCW;
     unsigned* err = p.d_err;
     const int pos = *glob(p.d_pos);
-    const int tok = min(max(*glob(p.d_token), 0), VOCAB - 1);
+    const int tok = min(max(p.token >= 0 ? p.token : *glob(p.d_token), 0), VOCAB - 1);
     const unsigned step = *glob(p.d_step);
     // Epochs start at 1: the arena starts zeroed, and a zero tag must never look current.
     const unsigned base = (step + 1u) * kEpochStride;
