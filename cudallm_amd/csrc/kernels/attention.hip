@@ -92,8 +92,7 @@ __global__ void __launch_bounds__(256) kv_write_kernel(const float* qkv, uint16_
 // running softmax (m, l, o), so the loop exchanges nothing between phases; they are merged once, at the wave's end,
 // then the workgroup's 8 waves in LDS.
 //
-// A kv head's tiles are dealt over its splits' waves as evenly as whole tiles allow, with only as many splits as give
-// every wave a tile: up to 256 tokens are one workgroup, which writes the output.  With more, each split publishes its
+// A kv head's tiles are dealt evenly to its splits' waves, with only as many splits as give every wave a tile: up to 256 tokens are one workgroup, which writes the output.  With more, each split publishes its
 // (o, m, l) as tagged words (value and tag in one 64-bit word, so a word that carries the tag carries the value) and the
 // last split's workgroup polls them and writes the output: one store-to-load hop instead of a second launch.
 //  * The workgroups it waits for have smaller indices and wait for nothing, so they have been dispatched before it and
@@ -101,8 +100,8 @@ __global__ void __launch_bounds__(256) kv_write_kernel(const float* qkv, uint16_
 //  * The tag is a NaN pattern with the launch's number, which scratch memory does not hold by accident, and the words
 //    are zeroed as they are consumed, so a replayed launch (same number) never meets its own earlier words.
 // Measured on MI355X, 8 kv heads, one call in a replayed graph of 16 (2 at 131071), before (128 tokens per workgroup
-// staged in LDS, a second kernel merging the splits one after the other) and now: 100 tokens 6.5 -> 5.3 us, 1000
-// 9.7 -> 7.7, 4000 18.4 -> 8.8, 8000 28.0 -> 11.0, 131071 375 -> 52 (5.1 TB/s).
+// staged in LDS, a second kernel merging the splits one after the other) and now: 100 tokens 6.5 -> 4.2 us, 1000
+// 9.7 -> 7.9, 4000 18.4 -> 9.0, 8000 28.0 -> 10.6, 131071 375 -> 52 (5.2 TB/s).
 // Workgroups in all: one per CU (2 waves per SIMD).  With workgroups of half the size, 512 measured 57 against 52 us
 // at 131071 tokens and 12.7 against 11.4 at 8000, 128 measured 82 and 11.7.
 constexpr int kSplitBlocks = 256;
@@ -280,30 +279,33 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
 #pragma unroll
             for (int i = 0; i < 4; ++i) qr[h][e + i] = v[i];
         }
-    const int ctx = *d_pos + 1;
     const int kvh = blockIdx.x, split = blockIdx.y, splits = gridDim.y;
-    const int tiles = (ctx + kTile - 1) / kTile, used = min(splits, (tiles + kWaves - 1) / kWaves);
-    if (split >= used) return;
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
     const int g = lane / 8, c = lane % 8;
-    // Tiles [t, end) of this wave; the last one may reach past ctx.
-    const unsigned wi = split * kWaves + w, waves = kWaves * used;
-    int t = static_cast<int>(static_cast<uint64_t>(wi) * tiles / waves);
-    const int end = static_cast<int>(static_cast<uint64_t>(wi + 1) * tiles / waves);
-
-    // A kv head's rows as a uniform base and the lane's offset from the wave's first row (32 bits: 2^24 rows of a wave).
-    const size_t first = (static_cast<size_t>(kvh) * max_seq + static_cast<size_t>(t) * kTile) * kHd;
-    const char* K = reinterpret_cast<const char*>(kc + first);
-    const char* V = reinterpret_cast<const char*>(vc + first);
-    const int t_first = t, last_row = ctx - 1 - t * kTile;
-    auto load = [&](KvTile& kv, int tile) {  // rows past ctx read the last row again
+    // A tile's first row as a uniform base, then the lane's offset; rows past `last` (in the tile) read that one again.
+    auto load = [&](KvTile& kv, int tile, int last) {
+        const size_t first = (static_cast<size_t>(kvh) * max_seq + static_cast<size_t>(tile) * kTile) * kHd;
+        const char* K = reinterpret_cast<const char*>(kc + first);
+        const char* V = reinterpret_cast<const char*>(vc + first);
 #pragma unroll
         for (int r = 0; r < kTileRows; ++r) {
-            const uint32_t off = min((tile - t_first) * kTile + 8 * r + g, last_row) * (kHd * 2) + c * 16;
+            const uint32_t off = min(8 * r + g, last) * (kHd * 2) + c * 16;
             kv.k[r] = load_stream(K + off);
             kv.v[r] = load_stream(V + off);
         }
     };
+    // Wave wi takes tile wi and then its share of the tiles past one for each wave, in one piece (dealt in turn, 60 against
+    // 53 us at 131071 tokens).  The first tile does not depend on *d_pos, so the first split's waves request theirs before
+    // it has arrived (rows of the cache past ctx weigh nothing), a memory round trip less for short contexts: 100 tokens
+    // 5.3 -> 4.1 us.  The other splits wait, for they may have nothing to do.
+    const int wi = split * kWaves + w;
+    KvTile A, B;
+    const bool early = split == 0 && (w + 1) * kTile <= max_seq;
+    if (early) load(A, wi, kTile - 1);
+    const int ctx = *d_pos + 1;
+    const int tiles = (ctx + kTile - 1) / kTile, used = min(splits, (tiles + kWaves - 1) / kWaves), waves = kWaves * used;
+    if (split >= used) return;
+    auto last_of = [&](int tile) { return ctx - 1 - tile * kTile; };
     Running st;
 #pragma unroll
     for (int h = 0; h < kGroup; ++h) {
@@ -312,28 +314,29 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
 #pragma unroll
         for (int e = 0; e < 8; ++e) st.o[h][e] = 0.f;
     }
-    if (t < end) {
-        auto step = [&](const KvTile& kv, int tile) {
-            attend(kv, qr, st, tile * kTile, g, ctx);
-        };
-        KvTile A, B;
-        load(A, t);
+    if (wi < tiles) {
+        auto step = [&](const KvTile& kv, int tile) { attend(kv, qr, st, tile * kTile, g, ctx); };
+        const uint64_t more = max(tiles - waves, 0);
+        int t = wi, next = waves + static_cast<int>(more * wi / waves);
+        const int end = waves + static_cast<int>(more * (wi + 1) / waves);
+        if (!early) load(A, t, last_of(t));
         for (;;) {
-            if (t + 1 >= end) {
+            if (next >= end) {
                 step(A, t);
                 break;
             }
-            load(B, t + 1);
+            load(B, next, last_of(next));
             __builtin_amdgcn_sched_barrier(0);  // the next tile's loads go out before this tile's math
             step(A, t);
-            if (++t + 1 >= end) {
+            t = next++;
+            if (next >= end) {
                 step(B, t);
                 break;
             }
-            load(A, t + 1);
+            load(A, next, last_of(next));
             __builtin_amdgcn_sched_barrier(0);
             step(B, t);
-            ++t;
+            t = next++;
         }
     }
 
