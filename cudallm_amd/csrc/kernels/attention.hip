@@ -85,112 +85,121 @@ __global__ void __launch_bounds__(256) kv_write_kernel(const float* qkv, uint16_
 // ---- split-K attention -------------------------------------------------------------------------------
 //
 // One kernel.  Bound by the K and V bytes at long contexts, by latency at short ones.  A wave takes whole 32-token
-// tiles: lane (g, c) = (lane / 8, lane % 8) loads 16 bytes, columns 8c .. 8c + 7, of tokens g, g + 8, g + 16 and g + 24,
-// so every load instruction reads 1 KiB of consecutive cache rows straight into registers (no LDS staging), and the next
-// tile's 8 KiB are in flight while this one is multiplied.  All 4 query heads of the kv head run on the same registers:
-// 8 mixed-precision FMAs per head and token, summed over the 8 column lanes by DPP.  Each token phase g keeps its own
-// running softmax (m, l, o), so the loop exchanges nothing between phases; they are merged once, at the wave's end,
-// then the workgroup's 8 waves in LDS.
+// tiles, straight from the cache into registers in the matrix instructions' layout (no LDS staging), with the next tile's
+// 8 KiB in flight while this one is multiplied.  Both products run on v_mfma_f32_16x16x32_f16: the 16 query rows are the kv
+// head's 4 query heads times up to 4 fp16 parts of a 32-bit value (11 bits each, three used), so the fp16 keys meet the
+// whole query and the fp16 values the whole weight, with products exact and sums in 32 bits.  The weights come out of the
+// first product in the lanes in which the second takes them, eight tokens a lane.  About 180 instructions per tile, against
+// 480 with mixed-precision FMAs and a sum over lanes per score: that form measured, in one call of a replayed graph, 4.3 us
+// at 100 tokens, 10.7 at 8000 and 52.8 at 131071, this one 4.1, 9.9 and 46.
 //
-// A kv head's tiles are dealt evenly to its splits' waves, with only as many splits as give every wave a tile: up to 256 tokens are one workgroup, which writes the output.  With more, each split publishes its
-// (o, m, l) as tagged words (value and tag in one 64-bit word, so a word that carries the tag carries the value) and the
-// last split's workgroup polls them and writes the output: one store-to-load hop instead of a second launch.
+// A kv head's tiles are dealt evenly to its splits' waves, with only as many splits as give every wave a tile: up to 256
+// tokens are one workgroup, which writes the output.  With more, each split publishes its (o, m, l) as tagged words (value
+// and tag in one 64-bit word, so a word that carries the tag carries the value) and the last split's workgroup polls them
+// and writes the output: one store-to-load hop instead of a second launch.
 //  * The workgroups it waits for have smaller indices and wait for nothing, so they have been dispatched before it and
 //    always finish.  The wait is bounded besides; should it run out, the outputs are NaN.
 //  * The tag is a NaN pattern with the launch's number, which scratch memory does not hold by accident, and the words
 //    are zeroed as they are consumed, so a replayed launch (same number) never meets its own earlier words.
 // Measured on MI355X, 8 kv heads, one call in a replayed graph of 16 (2 at 131071), before (128 tokens per workgroup
-// staged in LDS, a second kernel merging the splits one after the other) and now: 100 tokens 6.5 -> 4.2 us, 1000
-// 9.7 -> 7.9, 4000 18.4 -> 9.0, 8000 28.0 -> 10.6, 131071 375 -> 52 (5.2 TB/s).
-// Workgroups in all: one per CU (2 waves per SIMD).  With workgroups of half the size, 512 measured 57 against 52 us
-// at 131071 tokens and 12.7 against 11.4 at 8000, 128 measured 82 and 11.7.
+// staged in LDS, a second kernel merging the splits one after the other) and now: 100 tokens 6.5 -> 4.1 us, 1000
+// 9.7 -> 7.3, 4000 18.4 -> 8.4, 8000 28.0 -> 9.9, 131071 375 -> 46 (5.8 TB/s).
+// Workgroups in all: one per CU (2 waves per SIMD).  With the FMA form in workgroups of half the size, 512 measured 57
+// against 52 us at 131071 tokens and 12.7 against 11.4 at 8000, 128 measured 82 and 11.7.
 constexpr int kSplitBlocks = 256;
 constexpr int kMaxSplits = 64;     // splits of one kv head
 constexpr int kWaves = 8;          // per workgroup
 constexpr int kTile = 32;
-constexpr int kTileRows = kTile / 8;
 constexpr float kScore2 = 0.125f * 1.4426950408889634f;  // score scale times log2(e)
 
-struct KvTile {
-    u32x4 k[kTileRows], v[kTileRows];
-};
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-// The running softmax of one token phase: m, l and the lane's 8 output columns for each of the 4 heads, in powers of
-// two: m is the largest score times log2(e), a weight is exp2(score log2(e) - m) from one FMA on the raw dot product.
-// m starts at the lowest float, not -inf, so that a score of -inf (a cached -inf) weighs exp2(-inf) = 0 and not NaN.
-struct Running {
-    float m[kGroup], l[kGroup], o[kGroup][8];
+// A wave's 32 tokens as the matrix instructions take them.  k[a][s]: lane (n, g) = (lane % 16, lane / 16) holds columns
+// 32 s + 8 g .. + 7 of token 16 a + n.  v[j]: columns 4 n .. 4 n + 3 of token token_of(g, j).
+struct KvTile {
+    u32x4 k[2][2];
+    u32x2 v[8];
 };
+__device__ __forceinline__ int token_of(int g, int j) { return 16 * (j / 4) + 4 * g + j % 4; }
 
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
+// exp of the difference of two scores, from the dot products.
+__device__ __forceinline__ float weight_of(float dot, float m) { return exp2_hw((dot - m) * kScore2); }
 
-// Sum over the 8 column lanes of a token (every lane gets it).
-__device__ __forceinline__ float sum8(float v) {
-    v += dpp<kDppXor1>(v);
-    v += dpp<kDppXor2>(v);
-    return v + dpp<kDppHalfMirror>(v);
+// The leading 11 bits (toward zero) of two floats as fp16; the floats keep the rest, 2^11 times.
+constexpr float kPart = 2048.f;
+__device__ __forceinline__ uint32_t take_f16(float& x, float& y) {
+    const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, y));
+    x = fmaf(half_bits_to_float(static_cast<uint16_t>(h)), -kPart, x * kPart);
+    y = fmaf(half_bits_to_float(static_cast<uint16_t>(h >> 16)), -kPart, y * kPart);
+    return h;
+}
+// Part p of two floats written as h + m 2^-11 + l 2^-22 with fp16 h, m, l (p = 3: nothing): all 24 bits of a float between
+// 2^16 and 2^-24, and 2^-46 at the least, although fp16 itself ends at 2^-24.
+__device__ __forceinline__ uint32_t part_f16(float x, float y, int p) {
+    const uint32_t h = take_f16(x, y), m = take_f16(x, y), l = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, y));
+    return p == 0 ? h : p == 1 ? m : p == 2 ? l : 0u;
 }
 
-// Maximum and sum over the 8 token phases (lane bits 3, 4, 5).
-__device__ __forceinline__ float phase_max(float v) {
-    v = fmaxf(v, dpp<kDppRor8>(v));
-    return max_lanes_xor<32>(max_lanes_xor<16>(v));
-}
-__device__ __forceinline__ float phase_sum(float v) {
-    v += dpp<kDppRor8>(v);
-    v = sum_lanes_xor<16>(v);
-    return sum_lanes_xor<32>(v);
-}
+// The running softmax of the wave: lane (n, g) holds, for head n / 4, the largest dot product m (starting at the lowest
+// float) and its share l of the weights 2^kLift exp(score - largest), and in o[b][i] the sums of part i of head g's weights
+// times column 4 n + b.  kLift puts the largest weight at 2^15, so that a weight has all its bits down to 2^-39 of that.
+// Weights come from differences of dot products, so they keep their meaning however large the scores are.
+constexpr float kLift = 15.f;
+struct Running {
+    float m, l;
+    f32x4 o[4];
+};
 
-// One tile: tokens t0 + 8 r + g; those at or past ctx weigh nothing.
-__device__ __forceinline__ void attend(const KvTile& kv, const float (&q)[kGroup][8], Running& st, int t0, int g, int ctx) {
-    float s[kTileRows][kGroup];
+// One tile at token t0; tokens at or past ctx weigh nothing.  qb: the group's queries, part n % 4 of head n / 4 as fp16 (one
+// power-of-two scale per head); ps: that part's scale; sc: the score scale times log2(e) over the head's scale.
+__device__ __forceinline__ void attend(const KvTile& kv, const f16x8 (&qb)[2], float ps, float sc, Running& st, int t0, int n, int g, int ctx) {
+    // Scores of tokens 16 a + 4 g + i against (head, part) n; the parts' sum over the head's 4 lanes.
+    f32x4 d[2];
 #pragma unroll
-    for (int r = 0; r < kTileRows; ++r)
+    for (int a = 0; a < 2; ++a) {
+        d[a] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int h = 0; h < kGroup; ++h) {
-            float d = 0.f;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                d = fmaf(half_bits_to_float(static_cast<uint16_t>(kv.k[r][e])), q[h][2 * e], d);
-                d = fmaf(half_bits_to_float(static_cast<uint16_t>(kv.k[r][e] >> 16)), q[h][2 * e + 1], d);
-            }
-            s[r][h] = sum8(d);
-            if (t0 + 8 * r + g >= ctx) s[r][h] = -INFINITY;
-        }
-    float m[kGroup];
-    bool moved = false;
-#pragma unroll
-    for (int h = 0; h < kGroup; ++h) {
-        m[h] = st.m[h];
-#pragma unroll
-        for (int r = 0; r < kTileRows; ++r) m[h] = fmaxf(m[h], s[r][h] * kScore2);
-        moved = moved || m[h] > st.m[h];
+        for (int s = 0; s < 2; ++s) d[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, kv.k[a][s]), qb[s], d[a], 0, 0, 0);
     }
-    if (__any(moved)) {  // a new maximum somewhere in the wave: rare after a chunk's first tiles
+    float x[8];
 #pragma unroll
-        for (int h = 0; h < kGroup; ++h) {
-            const float f = exp2_hw(st.m[h] - m[h]);
-            st.m[h] = m[h];
-            st.l[h] *= f;
+    for (int j = 0; j < 8; ++j) x[j] = d[j / 4][j % 4] * ps;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) st.o[h][e] *= f;
-        }
+    for (int j = 0; j < 8; ++j) x[j] += dpp<kDppXor1>(x[j]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] += dpp<kDppXor2>(x[j]);
+    u32x2 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = kv.v[j];
+    if (t0 + kTile > ctx) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (t0 + token_of(g, j) >= ctx) x[j] = -INFINITY, v[j] = u32x2{0u, 0u};  // the cache there may hold anything
     }
+    float m = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+    m = fmaxf(st.m, max_lanes_xor<32>(max_lanes_xor<16>(m)));
+    if (__any(m > st.m)) {  // a new maximum: rare after a wave's first tiles
+        const float f = exp2_hw((st.m - m) * sc), fo = __shfl(f, 4 * g);
+        st.m = m;
+        st.l *= f;
 #pragma unroll
-    for (int r = 0; r < kTileRows; ++r) {
-        u32x4 v = kv.v[r];
-        if (t0 + 8 * r + g >= ctx) v = u32x4{0, 0, 0, 0};  // the row loaded in its place may hold an inf
+        for (int b = 0; b < 4; ++b) st.o[b] *= fo;
+    }
+    float l[8];
 #pragma unroll
-        for (int h = 0; h < kGroup; ++h) {
-            const float p = exp2_hw(fmaf(s[r][h], kScore2, -m[h]));
-            st.l[h] += p;
+    for (int j = 0; j < 8; ++j) l[j] = x[j] = exp2_hw(fmaf(x[j] - m, sc, kLift));
+    st.l += ((l[0] + l[1]) + (l[2] + l[3])) + ((l[4] + l[5]) + (l[6] + l[7]));
+    u32x4 w;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                st.o[h][2 * e] = fmaf(p, half_bits_to_float(static_cast<uint16_t>(v[e])), st.o[h][2 * e]);
-                st.o[h][2 * e + 1] = fmaf(p, half_bits_to_float(static_cast<uint16_t>(v[e] >> 16)), st.o[h][2 * e + 1]);
-            }
-        }
+    for (int i = 0; i < 4; ++i) w[i] = part_f16(x[2 * i], x[2 * i + 1], n % 4);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        u32x4 c;  // column 4 n + b of the 8 tokens
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_perm(v[2 * i + 1][b / 2], v[2 * i][b / 2], b % 2 ? 0x07060302u : 0x05040100u);
+        st.o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, c), st.o[b], 0, 0, 0);
     }
 }
 
@@ -252,8 +261,8 @@ __device__ __forceinline__ void merge_half(const Partials& p, int h, int splits,
             if (s0 + 2 * i < n) tag_store(po + static_cast<size_t>(s0 + 2 * i) * kHd, 0.f, 0);
         const float sm = mine && lane < kRound ? value_of(vm) : -FLT_MAX;
         const float sl_ = __shfl(value_of(vm), lane + kRound);
-        const float mn = fmaxf(m, wave_max(sm)), f = exp2_hw(m - mn);
-        const float e = mine && lane < kRound ? exp2_hw(sm - mn) : 0.f;
+        const float mn = fmaxf(m, wave_max(sm)), f = weight_of(m, mn);
+        const float e = mine && lane < kRound ? weight_of(sm, mn) : 0.f;
         m = mn;
         l = fmaf(l, f, wave_sum(mine && lane < kRound ? sl_ * e : 0.f));
         o *= f;
@@ -263,36 +272,58 @@ __device__ __forceinline__ void merge_half(const Partials& p, int h, int splits,
     }
 }
 
+// The wave's tiles (`first`, then [begin, end)) one token at a time, lane = column: the closed form term by term.
+__device__ __forceinline__ void attend_plain(const float* q, const uint16_t* K, const uint16_t* V, int first, int begin, int end, int ctx,
+                                             int lane, float (&so)[kGroup][kHd], float (&sml)[kGroup][2]) {
+#pragma unroll 1
+    for (int h = 0; h < kGroup; ++h) {
+        const float qh = q[h * kHd + lane];
+        float m = -FLT_MAX, l = 0.f, o = 0.f;
+#pragma unroll 1
+        for (int t = first; t < end; t = t < begin ? begin : t + 1) {
+#pragma unroll 1
+            for (int j = t * kTile; j < min((t + 1) * kTile, ctx); ++j) {
+                const float s = wave_sum(qh * half_bits_to_float(K[static_cast<size_t>(j) * kHd + lane]));
+                const float mn = fmaxf(m, s), f = weight_of(m, mn), p = exp2_hw(fmaf(s - mn, kScore2, kLift));
+                l = fmaf(l, f, p);
+                o = fmaf(p, half_bits_to_float(V[static_cast<size_t>(j) * kHd + lane]), o * f);
+                m = mn;
+            }
+        }
+        so[h][lane] = o;
+        if (lane == 0) sml[h][0] = m, sml[h][1] = l;
+    }
+}
+
 // grid (nkv, splits), block 512.
 __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* q, const uint16_t* kc, const uint16_t* vc,
                                                                    const int* d_pos, Partials part, float* out, int max_seq) {
     __shared__ float so[kWaves][kGroup][kHd];  // [wave][head][column]
     __shared__ float sml[kWaves][kGroup][2];   // [wave][head] m, l
 
-    // The group's 4 queries, the lane's 8 columns of each.
-    float qr[kGroup][8];
-#pragma unroll
-    for (int h = 0; h < kGroup; ++h)
-#pragma unroll
-        for (int e = 0; e < 8; e += 4) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(q + (blockIdx.x * kGroup + h) * kHd + threadIdx.x % 8 * 8 + e);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) qr[h][e + i] = v[i];
-        }
     const int kvh = blockIdx.x, split = blockIdx.y, splits = gridDim.y;
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
-    const int g = lane / 8, c = lane % 8;
-    // A tile's first row as a uniform base, then the lane's offset; rows past `last` (in the tile) read that one again.
-    auto load = [&](KvTile& kv, int tile, int last) {
+    const int n = lane % 16, g = lane / 16;
+    // The lane's 16 columns of query n / 4 (as KvTile's k), requested first.
+    float qv[2][8];
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(q + (kvh * kGroup + n / 4) * kHd + 32 * (i / 8) + 8 * g + i % 8);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) qv[i / 8][i % 8 + e] = v[e];
+    }
+    // A tile (whole tiles lie inside the cache: max_seq is a multiple of 128).
+    auto load = [&](KvTile& kv, int tile) {
         const size_t first = (static_cast<size_t>(kvh) * max_seq + static_cast<size_t>(tile) * kTile) * kHd;
         const char* K = reinterpret_cast<const char*>(kc + first);
         const char* V = reinterpret_cast<const char*>(vc + first);
+        const uint32_t ko = n * (kHd * 2) + g * 16, vo = 4 * g * (kHd * 2) + n * 8;
 #pragma unroll
-        for (int r = 0; r < kTileRows; ++r) {
-            const uint32_t off = min(8 * r + g, last) * (kHd * 2) + c * 16;
-            kv.k[r] = load_stream(K + off);
-            kv.v[r] = load_stream(V + off);
-        }
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) kv.k[a][s] = gload(reinterpret_cast<const u32x4*>(K + ko + a * 16 * kHd * 2 + s * 64));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) kv.v[j] = __builtin_nontemporal_load((const __attribute__((address_space(1))) u32x2*)(V + vo + token_of(0, j) * (kHd * 2)));
     };
     // Wave wi takes tile wi and then its share of the tiles past one for each wave, in one piece (dealt in turn, 60 against
     // 53 us at 131071 tokens).  The first tile does not depend on *d_pos, so the first split's waves request theirs before
@@ -301,31 +332,40 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
     const int wi = split * kWaves + w;
     KvTile A, B;
     const bool early = split == 0 && (w + 1) * kTile <= max_seq;
-    if (early) load(A, wi, kTile - 1);
+    if (early) load(A, wi);
     const int ctx = *d_pos + 1;
     const int tiles = (ctx + kTile - 1) / kTile, used = min(splits, (tiles + kWaves - 1) / kWaves), waves = kWaves * used;
     if (split >= used) return;
-    auto last_of = [&](int tile) { return ctx - 1 - tile * kTile; };
-    Running st;
-#pragma unroll
-    for (int h = 0; h < kGroup; ++h) {
-        st.m[h] = -FLT_MAX;
-        st.l[h] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) st.o[h][e] = 0.f;
-    }
+    const uint64_t more = max(tiles - waves, 0);
+    const int begin = waves + static_cast<int>(more * wi / waves), end = waves + static_cast<int>(more * (wi + 1) / waves);
+    Running st{-FLT_MAX, 0.f, {}};
+    float m_dot = -FLT_MAX;  // st.m without the query's scale
     if (wi < tiles) {
-        auto step = [&](const KvTile& kv, int tile) { attend(kv, qr, st, tile * kTile, g, ctx); };
-        const uint64_t more = max(tiles - waves, 0);
-        int t = wi, next = waves + static_cast<int>(more * wi / waves);
-        const int end = waves + static_cast<int>(more * (wi + 1) / waves);
-        if (!early) load(A, t, last_of(t));
+        if (!early) load(A, wi);
+        __builtin_amdgcn_sched_barrier(0);
+        // The query's fp16 parts: the head's largest |q| scaled to 2^14 .. 2^15.
+        float big = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) big = fmaxf(big, fabsf(qv[i / 8][i % 8]));
+        big = max_lanes_xor<32>(max_lanes_xor<16>(big));
+        const int e = big > 0.f && big < INFINITY ? min(max(14 - ilogbf(big), -110), 110) : 0;
+        f16x8 qb[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            u32x4 p;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[i] = part_f16(ldexpf(qv[s][2 * i], e), ldexpf(qv[s][2 * i + 1], e), n % 4);
+            qb[s] = __builtin_bit_cast(f16x8, p);
+        }
+        const float sc = ldexpf(kScore2, -e), ps = ldexpf(1.f, -11 * (n % 4));
+        auto step = [&](const KvTile& kv, int tile) { attend(kv, qb, ps, sc, st, tile * kTile, n, g, ctx); };
+        int t = wi, next = begin;
         for (;;) {
             if (next >= end) {
                 step(A, t);
                 break;
             }
-            load(B, next, last_of(next));
+            load(B, next);
             __builtin_amdgcn_sched_barrier(0);  // the next tile's loads go out before this tile's math
             step(A, t);
             t = next++;
@@ -333,41 +373,24 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
                 step(B, t);
                 break;
             }
-            load(A, next, last_of(next));
+            load(A, next);
             __builtin_amdgcn_sched_barrier(0);
             step(B, t);
             t = next++;
         }
+        m_dot = ldexpf(st.m, -e);
     }
-
-    // The wave's 8 token phases: every phase is rescaled to the head's maximum, then summed by exchanges that halve the
-    // values a lane holds: lane bits 5 and 4 pick the head, bit 3 the half of the lane's 8 columns.
-    float M[kGroup];
+    st.l = sum_lanes_xor<32>(sum_lanes_xor<16>(st.l));
+    f32x4 y;  // columns 4 n .. 4 n + 3 of head g
 #pragma unroll
-    for (int h = 0; h < kGroup; ++h) {
-        M[h] = phase_max(st.m[h]);
-        const float f = exp2_hw(st.m[h] - M[h]);
-        st.l[h] = phase_sum(st.l[h] * f);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) st.o[h][e] *= f;
-    }
-    float x[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-        x[e] = fold_lanes<16>(fold_lanes<32>(st.o[0][e], st.o[1][e]), fold_lanes<32>(st.o[2][e], st.o[3][e]));
-    const bool odd = lane & 8;
-    f32x4 y;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] = (odd ? x[e + 4] : x[e]) + dpp<kDppRor8>(odd ? x[e] : x[e + 4]);
-    *reinterpret_cast<f32x4*>(&so[w][(lane >> 5) + 2 * ((lane >> 4) & 1)][c * 8 + (odd ? 4 : 0)]) = y;
-    if (lane < kGroup) {
-        float m = M[0], l = st.l[0];
-#pragma unroll
-        for (int h = 1; h < kGroup; ++h)
-            if (lane == h) m = M[h], l = st.l[h];
-        sml[w][lane][0] = m;
-        sml[w][lane][1] = l;
-    }
+    for (int b = 0; b < 4; ++b) y[b] = fmaf(fmaf(st.o[b][2], 1.f / kPart, st.o[b][1]), 1.f / kPart, st.o[b][0]);
+    *reinterpret_cast<f32x4*>(&so[w][g][4 * n]) = y;
+    if (g == 0 && n % 4 == 0) sml[w][n / 4][0] = m_dot, sml[w][n / 4][1] = st.l;
+    // An infinity or NaN among the inputs (or a score past the floats) leaves one here, as its parts do not add up to it:
+    // such a wave starts over with plain products.
+    if (__any(!(fabsf(m_dot) < INFINITY) || !(fabsf(st.l) < INFINITY) || !(fabsf((y[0] + y[1]) + (y[2] + y[3])) < INFINITY)))
+        attend_plain(q + kvh * kGroup * kHd, kc + static_cast<size_t>(kvh) * max_seq * kHd, vc + static_cast<size_t>(kvh) * max_seq * kHd,
+                     wi, begin, end, ctx, lane, so[w], sml[w]);
     __syncthreads();
 
     // Waves 0-3 take a head each: the 8 waves' partials in wave order.
@@ -378,7 +401,7 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
         for (int i = 0; i < kWaves; ++i) m = fmaxf(m, sml[i][w][0]);
 #pragma unroll
         for (int i = 0; i < kWaves; ++i) {
-            const float f = exp2_hw(sml[i][w][0] - m);
+            const float f = weight_of(sml[i][w][0], m);
             l = fmaf(sml[i][w][1], f, l);
             o = fmaf(so[i][w][lane], f, o);
         }
@@ -401,7 +424,7 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
     __syncthreads();
     if (w < kGroup) {
         const float m1 = sml[w + kGroup][0][0], l1 = sml[w + kGroup][0][1], o1 = so[w + kGroup][0][lane];
-        const float M = fmaxf(fmaxf(om, m1), m), f0 = exp2_hw(om - M), f1 = exp2_hw(m1 - M), f = exp2_hw(m - M);
+        const float M = fmaxf(fmaxf(om, m1), m), f0 = weight_of(om, M), f1 = weight_of(m1, M), f = weight_of(m, M);
         out[h * kHd + lane] = (oo * f0 + o1 * f1 + o * f) / (ol * f0 + l1 * f1 + l * f);
     }
 }

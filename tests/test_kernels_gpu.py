@@ -332,6 +332,42 @@ def test_attention_replayed_launch():
         assert torch.equal(out, want), f"ctx {ctx}"
 
 
+@pytest.mark.parametrize("case", ["small weights", "small query", "tiny query", "large query", "large keys"])
+def test_attention_dynamic_range(case):
+    """Terms far below the largest keep their bits: tokens whose weights are 2^-31 of one that adds nothing, query
+    columns 2^-30 of one that meets zeros, queries near the ends of the floats, keys at the end of fp16.  Against 64
+    bits within 1e-4 of the result (a weight's exponent carries the rounding of a score of up to 1e3 or so: 6e-5)."""
+    import torch
+    nkv, max_seq, ctx = 2, 2048, 1900
+    g = torch.Generator(device="cuda")
+    g.manual_seed(17)
+    q = torch.randn(nkv, 4, 64, generator=g, device="cuda")
+    k, v = (torch.randn(nkv, max_seq, 64, generator=g, device="cuda").half() for _ in range(2))
+    if case == "small weights":
+        q[..., 0], q[..., 1:] = 16.0, 0.01
+        k[..., 0] = 0.0
+        k[:, 700, 0], v[:, 700] = 0.125 ** -1 * 21.5 / 16, 0.0  # e^21.5 = 2^31
+    elif case == "small query":
+        q[..., 0] = 2.0 ** 30
+        k[..., 0] = 0.0
+    elif case == "tiny query":
+        q *= 1e-38
+    elif case == "large query":
+        q *= 1e37
+        k[:] = k[:, :1] * 1e-3  # equal scores: a uniform average
+    else:
+        k.mul_(15000.0).clamp_(-65504.0, 65504.0)
+        q *= 1e-4
+    pos = torch.tensor([ctx - 1], dtype=torch.int32, device="cuda")
+    out = torch.empty(nkv * 256, device="cuda")
+    E.launch_attention_static(q.data_ptr(), k.data_ptr(), v.data_ptr(), pos.data_ptr(), out.data_ptr(), 4 * nkv, nkv, 64,
+                              max_seq, torch.cuda.current_stream().cuda_stream)
+    s = torch.matmul(q.double().cpu(), k[:, :ctx].double().cpu().transpose(1, 2)) * 0.125
+    p = torch.softmax(torch.zeros_like(s) if case == "large query" else s, dim=-1)
+    ref = torch.matmul(p, v[:, :ctx].double().cpu()).view(-1)
+    assert (out.double().cpu() - ref).norm() <= 1e-4 * ref.norm()
+
+
 @pytest.mark.parametrize("where", ["k", "v", "q"])
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
 def test_attention_non_finite(where, value):
