@@ -61,6 +61,26 @@ __device__ __forceinline__ void store_out(float* y, int r, float d, float du) {
     }
 }
 
+// The fixed-point scale of the digits here fills the digits' whole range (|xi| up to about 2^23, a bit more than digits.h's
+// own words hold), so that the rounding of x^ adds no more than the sums in 32 bits did: 24576 x 4096 int4 with SWIGLU,
+// against 64 bits: 5.1e-7 converting every weight, 8.1e-7 with |xi| < 2^22, 4.2e-7 so.
+template <WType WT>
+__device__ __forceinline__ int wide_exponent(float m) {
+    if (!(m > 0.f) || !(m < INFINITY)) return 0;
+    constexpr float kMost = WT == WType::INT8 ? 8355700.f : 7829350.f;  // 127 (1 + 256 + 256^2), 7 (1 + 16 + ... + 16^5)
+    const int e = min(22 - ilogbf(m), 126);
+    return ldexpf(m, e) > kMost ? e - 1 : e;
+}
+__device__ __forceinline__ uint32_t wide_word(float v, float scale, uint32_t C) {
+    return static_cast<uint32_t>(static_cast<int>(rintf(v * scale))) + C;
+}
+
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+__device__ __forceinline__ Rsrc make_rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+constexpr int kAuxNt = 2;  // non-temporal
+
 template <WType WT, Epilogue EP, bool NORM, int KS, int R>
 __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     using F = Fmt<WT>;
@@ -70,6 +90,10 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     constexpr bool GLU = EP == Epilogue::SWIGLU;
     constexpr int NP = GLU ? 2 : 1;
     constexpr bool DIG = WT != WType::BF16 && KS == 1;
+    // x^ by lines of 64 chunks, a lane's 16-byte words of a line at [line][word][lane]: the digits of a chunk, or its
+    // floats.  One copy with KS = 1, a slice per wave with KS > 1.
+    constexpr int XW = !DIG ? F::CPC / 4 : WT == WType::INT4 ? 6 : 3;
+    __shared__ u32x4 xs[KS][F::CPL * XW * kWave];
     __shared__ float scratch[16];
     __shared__ float part[KS > 1 ? KS * ROWS_WG * NP : 1];
 
@@ -86,18 +110,19 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     if (base >= out_rows) return;
     int left = (out_rows - base + stride - 1) / stride;  // passes of this workgroup, >= 1
 
-    // The lane's 32 inputs (and norm weights) are requested first, then the first pass's weights, so that the
-    // prologue below waits only for the short input loads while the weight bytes are already in flight (loads
-    // complete in order, so requesting the weights first would make the prologue wait for them).
-    f32x4 xin[NX / 4], nwin[NORM ? NX / 4 : 1];
+    // The inputs (and norm weights) are requested first, then the first pass's weights, so that the prologue below waits
+    // only for the short input loads while the weight bytes are already in flight (loads complete in order, so requesting
+    // the weights first would make the prologue wait for them).  They are read in consecutive 16-byte words and change
+    // hands in LDS: with KS = 1 thread t takes columns 8 t .. 8 t + 7 of the row that all four waves share, with KS > 1 a
+    // wave takes its own slice.  Read the way the lanes use them (32 columns at a stride of 32 to 128 bytes, by every
+    // wave), each load touched up to 64 lines: int4 512 x 2048 4.3 us against 2.8 for bf16.
+    constexpr int XV = KS == 1 ? 2 : NX / 4;
+    f32x4 xin[XV], nwin[NORM ? XV : 1];
 #pragma unroll
-    for (int k = 0; k < F::CPL; ++k) {
-        const int c0 = slice * kSlice + (k * kWave + lane) * F::CPC;
-#pragma unroll
-        for (int j = 0; j < F::CPC; j += 4) {
-            xin[(k * F::CPC + j) / 4] = *reinterpret_cast<const f32x4*>(a.x + c0 + j);
-            if constexpr (NORM) nwin[(k * F::CPC + j) / 4] = *reinterpret_cast<const f32x4*>(a.norm_w + c0 + j);
-        }
+    for (int i = 0; i < XV; ++i) {
+        const int j = KS == 1 ? 2 * tid + i : slice * (kSlice / 4) + i * kWave + lane;
+        xin[i] = reinterpret_cast<const f32x4*>(a.x)[j];
+        if constexpr (NORM) nwin[i] = reinterpret_cast<const f32x4*>(a.norm_w)[j];
     }
     const size_t rb = row_bytes<WT>(a.cols);
     // Addresses are a row base that is uniform across the wave (scalar registers) plus a 32-bit lane offset, the
@@ -139,68 +164,95 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     load(A, base + grp * R);
     __builtin_amdgcn_sched_barrier(0);  // keep the weight loads ahead of the prologue
 
-    // RMSNorm: with KS = 1 every wave holds the whole row (64 lanes x 32 columns), so a wave sum gives the sum of
-    // squares; with KS > 1 the workgroup's waves hold one slice each.
+    // RMSNorm's sum of squares and, for the digits, the largest |x norm_w| (infinite if any input is infinite or NaN).
     float inv = 1.f;
-    if constexpr (NORM) {
-        float ss = 0.f;
+    [[maybe_unused]] float dsc = 1.f, scale = 1.f;
+    if constexpr (NORM || DIG) {
+        float ss = 0.f, mx = 0.f;
 #pragma unroll
-        for (int q = 0; q < NX / 4; ++q)
-            ss += xin[q][0] * xin[q][0] + xin[q][1] * xin[q][1] + xin[q][2] * xin[q][2] + xin[q][3] * xin[q][3];
-        ss = KS == 1 ? wave_sum(ss) : block_sum(ss, scratch);
-        inv = rsqrtf(ss / static_cast<float>(a.cols) + a.eps);
-    }
-    float xr[NX];
-    float xsum = 0.f;
+        for (int q = 0; q < XV; ++q)
 #pragma unroll
-    for (int q = 0; q < NX / 4; ++q) {
-        f32x4 v = xin[q];
+            for (int e = 0; e < 4; ++e) {
+                ss = fmaf(xin[q][e], xin[q][e], ss);
+                if constexpr (DIG) {
+                    const float t = fabsf(NORM ? xin[q][e] * nwin[q][e] : xin[q][e]);
+                    mx = t < INFINITY ? fmaxf(mx, t) : INFINITY;
+                }
+            }
+        if constexpr (NORM) ss = wave_sum(ss);
+        if constexpr (DIG) mx = wave_max(mx);
+        if (lane == 0) scratch[wave] = ss, scratch[4 + wave] = mx;
+        __syncthreads();
         if constexpr (NORM) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = v[e] * inv * nwin[q][e];
+            ss = ((scratch[0] + scratch[1]) + scratch[2]) + scratch[3];
+            inv = rsqrtf(ss / static_cast<float>(a.cols) + a.eps);
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            xr[4 * q + e] = v[e];
-            xsum += v[e];
+        if constexpr (DIG) {
+            mx = fmaxf(fmaxf(scratch[4], scratch[5]), fmaxf(scratch[6], scratch[7])) * inv;
+            const int e = wide_exponent<WT>(mx);
+            scale = ldexpf(1.f, e);
+            dsc = mx < INFINITY ? ldexpf(1.f, -e) : __builtin_nanf("");
         }
+    }
+    if constexpr (NORM)
+#pragma unroll
+        for (int q = 0; q < XV; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xin[q][e] = xin[q][e] * inv * nwin[q][e];
+    if constexpr (DIG) {
+        // Digit words of the thread's 8 columns in the weight words' layout.
+        uint32_t* const xw = reinterpret_cast<uint32_t*>(xs[0]);
+        if constexpr (WT == WType::INT8) {
+            const int at = (tid / 2 / kWave * XW * kWave + tid / 2 % kWave) * 4 + tid % 2 * 2;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                uint32_t P[3];
+                byte_planes(wide_word(xin[h][0], scale, 0x808080u), wide_word(xin[h][1], scale, 0x808080u),
+                            wide_word(xin[h][2], scale, 0x808080u), wide_word(xin[h][3], scale, 0x808080u), P);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) xw[at + d * kWave * 4 + h] = P[d] ^ 0x80808080u;
+            }
+        } else {
+            uint32_t u[8], w[6];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) u[e] = wide_word(xin[e / 4][e % 4], scale, 0x888888u);
+            nibble_words(u, w);
+#pragma unroll
+            for (int d = 0; d < 6; ++d) xw[d * kWave * 4 + tid] = w[d] ^ 0x88888888u;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < XV; ++i) {
+            const int j = KS == 1 ? 2 * tid + i : i * kWave + lane, c = j / XW;
+            xs[KS == 1 ? 0 : slice][(c / kWave * XW + j % XW) * kWave + c % kWave] = __builtin_bit_cast(u32x4, xin[i]);
+        }
+    }
+    if constexpr (KS == 1) {
+        __syncthreads();
+    } else {  // a wave reads what it wrote
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 
-    // Digit words of the lane's inputs in its weight words' layout: int8 digit k of chunk c, word t (columns
-    // 4t .. 4t + 3) at dg[(2k + c) 4 + t]; int4 digit k of word t (columns 8t .. 8t + 7) at dg[4k + t].
+    // The lane's inputs: digit words (int8 digit k of chunk c, word t (columns 4t .. 4t + 3) at dg[(2k + c) 4 + t]; int4
+    // digit k of word t (columns 8t .. 8t + 7) at dg[4k + t]) or 32 floats and their sum.
     [[maybe_unused]] uint32_t dg[DIG ? 24 : 1];
-    [[maybe_unused]] float dsc = 1.f;
-    if constexpr (DIG) {
-        float m = 0.f;
+    [[maybe_unused]] float xr[DIG ? 1 : NX], xsum = 0.f;
 #pragma unroll
-        for (int j = 0; j < NX; ++j) m = fmaxf(m, fabsf(xr[j]));
-        const int e = dig_exponent(wave_max(m));
-        dsc = ldexpf(1.f, -e);
-        const float scale = ldexpf(1.f, e);
-        if constexpr (WT == WType::INT8) {
+    for (int k = 0; k < F::CPL; ++k)
 #pragma unroll
-            for (int c = 0; c < 2; ++c)
+        for (int q = 0; q < XW; ++q) {
+            const u32x4 v = xs[KS == 1 ? 0 : slice][(k * XW + q) * kWave + lane];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const float* xc = xr + c * 16 + 4 * t;
-                    uint32_t P[3];
-                    byte_planes(fixed_word(xc[0], scale, 0x808080u), fixed_word(xc[1], scale, 0x808080u),
-                                fixed_word(xc[2], scale, 0x808080u), fixed_word(xc[3], scale, 0x808080u), P);
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) dg[(2 * k + c) * 4 + t] = P[k] ^ 0x80808080u;
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (DIG) {
+                    dg[(q * F::CPL + k) * 4 + e] = v[e];
+                } else {
+                    xr[k * F::CPC + 4 * q + e] = __builtin_bit_cast(f32x4, v)[e];
+                    xsum += xr[k * F::CPC + 4 * q + e];
                 }
-        } else {
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                uint32_t u[8], w[6];
-#pragma unroll
-                for (int b = 0; b < 8; ++b) u[b] = fixed_word(xr[8 * t + b], scale, 0x888888u);
-                nibble_words(u, w);
-#pragma unroll
-                for (int k = 0; k < 6; ++k) dg[4 * k + t] = w[k] ^ 0x88888888u;
             }
         }
-    }
 
     // KS = 1: the row sums wait in lanes (lane j: the wave's j-th row) and are stored after the last pass, so no store
     // sits in the loop (a store there made the loop's head wait for the previous pass's loads).  The host keeps every
@@ -375,26 +427,6 @@ constexpr int kXPairs = 12288 / 8 / kWideThreads;  // a thread stages 8 columns 
 // 13.2 / 14.2; 1000 x 1024: bf16 3.1 / 3.1 / 3.5, int8 3.4 / 3.5 / 3.9, int4 3.6 / 4.0 / 4.2.
 template <WType WT>
 constexpr int kDepth = WT == WType::INT4 ? 2 : 3;
-
-// The fixed-point scale here fills the digits' whole range (|xi| up to about 2^23, a bit more than digits.h's own words
-// hold), so that the rounding of x^ adds no more than the sums in 32 bits did: 24576 x 4096 int4 with SWIGLU, against 64
-// bits: 5.1e-7 converting every weight, 8.1e-7 with |xi| < 2^22.
-template <WType WT>
-__device__ __forceinline__ int wide_exponent(float m) {
-    if (!(m > 0.f) || !(m < INFINITY)) return 0;
-    constexpr float kMost = WT == WType::INT8 ? 8355700.f : 7829350.f;  // 127 (1 + 256 + 256^2), 7 (1 + 16 + ... + 16^5)
-    const int e = min(22 - ilogbf(m), 126);
-    return ldexpf(m, e) > kMost ? e - 1 : e;
-}
-__device__ __forceinline__ uint32_t wide_word(float v, float scale, uint32_t C) {
-    return static_cast<uint32_t>(static_cast<int>(rintf(v * scale))) + C;
-}
-
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-__device__ __forceinline__ Rsrc make_rsrc(const void* p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
-}
-constexpr int kAuxNt = 2;  // non-temporal
 
 template <WType WT>
 struct Wide {
