@@ -7,9 +7,9 @@
 //    one row (one slice each), so the 4 waves of a workgroup cover 4/KS row groups.
 //  * Every lane owns a fixed set of 32 columns of its slice: the 16-byte chunks lane, lane+64, ...
 //    (8 bf16 / 16 int8 / 32 int4 columns per chunk).  Those 32 inputs - normalised when the norm
-//    is fused - are loaded ONCE into VGPRs and reused for every row the wave touches, so the inner
-//    loop reads no LDS at all: only 128-bit non-temporal weight loads, 64 lanes x 16 B = 1 KiB
-//    contiguous per load instruction.
+//    is fused - are read and normalised once per workgroup, handed to the lanes through LDS and kept in
+//    VGPRs for every row the wave touches, so the inner loop reads no LDS at all: only 128-bit
+//    non-temporal weight loads, 64 lanes x 16 B = 1 KiB contiguous per load instruction.
 //  * R rows (rpb) are loaded before any is consumed, for R x (4 KiB bf16 | 2 KiB int8 | 1 KiB int4)
 //    of loads per pass; a wave issues the next pass's loads before it multiplies the current one,
 //    so up to 2R rows are in flight.  The first pass's weights are requested right after the lane's
@@ -19,9 +19,8 @@
 //    pass also waited for the next pass's loads.  Measured on MI355X against the earlier form: lm_head
 //    bf16 82.5 -> 80.0 us, int8 44.6 -> 40.5 us, int4 32.2 -> 28.0 us; bf16 and int8 lm_head then run
 //    within 1 % of a plain stream read of the same bytes.
-//  * Quantised 2048-wide rows (KS = 1) use integer digit dots: each lane turns its 32 inputs into
-//    fixed-point digit words once (one scale per wave from max |x^|, the same in every wave since each
-//    covers the whole row), and a row then costs 24 v_dot8_i32_i4 / v_dot4_i32_i8 per lane instead of
+//  * Quantised 2048-wide rows (KS = 1) use integer digit dots: the workgroup turns the inputs into
+//    fixed-point digit words once (one scale from max |x^|), and a row then costs 24 v_dot8_i32_i4 / v_dot4_i32_i8 per lane instead of
 //    a conversion and an FMA per column.  The 8192-wide down rows (KS = 4) keep the float path.
 //  * Row sums are wave64 DPP butterflies (deterministic order); with KS > 1 the slice partials
 //    meet in LDS and are added in slice order.  No atomics anywhere.
@@ -29,7 +28,7 @@
 //    many as can be resident)), but with KS = 1 at least enough workgroups that none takes more than
 //    64 / R passes.
 //
-// Widths other than 2048 and 8192 use matvec_wide, which stages x in LDS.
+// Widths other than 2048 and 8192 (and some of 8192, see pick_shape) use matvec_wide, which stages x in LDS.
 #pragma once
 
 #include <algorithm>
@@ -712,7 +711,11 @@ void pick_r(int rpb, const MatvecArgs& a, hipStream_t s) {
 template <WType WT, Epilogue EP, bool NORM>
 void pick_shape(int rpb, const MatvecArgs& a, hipStream_t s) {
     if (a.cols == 2048) return pick_r<WT, EP, NORM, 1>(rpb, a, s);
-    if (a.cols == 8192) return pick_r<WT, EP, NORM, 4>(rpb, a, s);
+    // Quantised 8192-wide rows convert every weight in matvec_fast, for want of columns per wave to share the digits of
+    // x^ with; with two matrices of many rows the any-width kernel's digits are faster: SWIGLU rows 4096 / 8192 / 30000, int4
+    // 8.8 / 13.2 / 38.9 -> 7.7 / 11.0 / 25.6 us, int8 9.3 / 15.6 / 47.7 -> 9.2 / 14.5 / 45.3.  Without SWIGLU matvec_fast
+    // stays ahead at most row counts (2048: int4 5.1 against 6.2, int8 5.7 against 6.6; 16384: int8 26.2 against 27.1).
+    if (a.cols == 8192 && !(WT != WType::BF16 && EP == Epilogue::SWIGLU && a.rows >= 4096)) return pick_r<WT, EP, NORM, 4>(rpb, a, s);
     return launch_wide<WT, EP, NORM>(a, s);
 }
 

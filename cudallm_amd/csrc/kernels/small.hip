@@ -31,19 +31,20 @@ int device_cu_count() {
 //
 // kDefaultRpb is the rpb used when the caller passes 0.  kGridPerCu caps the grid at that many workgroups per CU
 // (0: as many as can be resident at once).  Smaller grids mean fewer workgroups, each with more passes, so fewer
-// repeats of the input and norm prologue; for bf16 lm_head a grid of 16 workgroups per CU, more than can be resident
-// at once, spreads the last passes more evenly.  Measured effects: bf16 qkv 4.69 -> 4.40 us, gate_up 12.50 -> 12.00,
-// down 7.65 -> 7.50, lm_head 79.8 -> 78.0 (8 per CU) -> 77.0 (16); int8 gate_up 8.53 -> 7.25; int4 gate_up
-// 7.72 -> 6.68, lm_head 26.50 -> 25.28.
+// repeats of the input and norm prologue; larger ones than can be resident spread the last passes more evenly over
+// many rows.  Measured effects: bf16 qkv 4.69 -> 4.40 us, gate_up 12.50 -> 12.00, down 7.65 -> 7.50, lm_head
+// 79.8 -> 78.0 (8 per CU) -> 77.0 (16); int8 gate_up 8.53 -> 7.25, down 5.94 -> 5.77 (rpb 4 -> 2, 2 per CU), lm_head
+// 43.6 -> 42.0 (8 per CU), 20483 x 2048 9.05 -> 8.76 (2 per CU); int4 gate_up 7.72 -> 6.68, lm_head 24.3 -> 23.4
+// (2 -> 8 per CU), 20483 x 2048 6.67 -> 6.04 (2 per CU).
 constexpr int kDefaultRpb[3][4] = {
     {1, 1, 2, 2},  // bf16
-    {4, 2, 4, 4},  // int8
-    {4, 4, 8, 4},  // int4
+    {4, 2, 2, 4},  // int8
+    {4, 4, 4, 4},  // int4
 };
 constexpr int kGridPerCu[3][4] = {
     {1, 1, 2, 16},  // bf16
-    {0, 1, 0, 0},   // int8
-    {0, 1, 0, 2},   // int4
+    {2, 1, 2, 8},   // int8
+    {2, 1, 2, 8},   // int4
 };
 
 namespace {
@@ -59,7 +60,23 @@ int type_index(WType wt) {
 }
 }  // namespace
 
-int default_rpb(WType wt, Epilogue ep, int rows, int cols) { return kDefaultRpb[type_index(wt)][shape_class(ep, rows, cols)]; }
+// The class's rpb, adjusted to the row count on 256 CUs:
+//  * Few rows of class 0 are spread over more workgroups: rpb is halved while they (4 waves of rpb rows each) would fill
+//    less than half of the CUs.  1500 x 2048: int8 3.06 -> 2.71 us, int4 2.83 -> 2.67; 512 rows: 2.89 -> 2.54, 2.77 -> 2.55.
+//  * Quantised rows of 8192 columns: each workgroup (rpb rows) reads 32 KiB of inputs, so rpb is doubled, up to 4 (int8) or
+//    8 (int4), as far as that gets by with one workgroup per CU: 700 rows int8 with norm 5.0 -> 4.0 us; 1100 rows int4 5.0
+//    -> 4.9.  More rows than that take the class's own: 2600 rows int8 6.6 against 6.9 with 4, int4 5.9 against 7.0 with 8.
+int default_rpb(WType wt, Epilogue ep, int rows, int cols) {
+    const int c = shape_class(ep, rows, cols), base = kDefaultRpb[type_index(wt)][c];
+    int r = base;
+    if (c == 0)
+        while (r > 1 && rows < 128 * 4 * r) r /= 2;
+    if (c == 2 && wt != WType::BF16) {
+        while (r < 2 * base && rows > 256 * r) r *= 2;
+        if (rows > 256 * r) r = base;
+    }
+    return r;
+}
 
 int grid_per_cu(WType wt, Epilogue ep, int rows, int cols) { return kGridPerCu[type_index(wt)][shape_class(ep, rows, cols)]; }
 

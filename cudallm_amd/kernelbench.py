@@ -27,13 +27,22 @@ RPBS = (1, 2, 4, 8)
 # The library's choice when rpb = 0 (kDefaultRpb / default_rpb in csrc/kernels/small.hip), and its grid size in
 # workgroups per CU (kGridPerCu; 0: as many as can be resident), per weight type and shape class: other, SwiGLU, 8192
 # columns, >= 65536 rows.
-DEFAULT_RPB = {"bf16": (1, 1, 2, 2), "int8": (4, 2, 4, 4), "int4": (4, 4, 8, 4)}
-GRID_PER_CU = {"bf16": (1, 1, 2, 16), "int8": (0, 1, 0, 0), "int4": (0, 1, 0, 2)}
+DEFAULT_RPB = {"bf16": (1, 1, 2, 2), "int8": (4, 2, 2, 4), "int4": (4, 4, 4, 4)}
+GRID_PER_CU = {"bf16": (1, 1, 2, 16), "int8": (2, 1, 2, 8), "int4": (2, 1, 2, 8)}
 
 
 def default_rpb(wd: str, ep: str, rows: int, cols: int) -> int:
     cls = 1 if ep == "swiglu" else 2 if cols >= 8192 else 3 if rows >= 65536 else 0
-    return DEFAULT_RPB[wd][cls]
+    base = r = DEFAULT_RPB[wd][cls]
+    if cls == 0:  # few rows: spread over more workgroups
+        while r > 1 and rows < 128 * 4 * r:
+            r //= 2
+    elif cls == 2 and wd != "bf16":  # twice the rows per workgroup where that makes one workgroup per CU do
+        if 256 * r < rows <= 512 * r:
+            r = 2 * base
+    return r
+
+
 PEAK_GBPS = 8000.0
 
 

@@ -102,10 +102,13 @@ def test_matvec_generic_and_ragged(wtype, rows, cols, epilogue):
 
 @pytest.mark.parametrize("wtype", ["bf16", "int8", "int4"])
 @pytest.mark.parametrize("rows,cols,epilogue", [(1, 1024, "store"), (3, 5120, "add"), (2, 11264, "swiglu"),
-                                                (8191, 1024, "store"), (8194, 7168, "swiglu"), (600000, 1024, "store")])
+                                                (8191, 1024, "store"), (8194, 7168, "swiglu"), (600000, 1024, "store"),
+                                                (4094, 8192, "swiglu"), (4098, 8192, "swiglu"), (513, 2048, "store"),
+                                                (1025, 2048, "add"), (1025, 8192, "add")])
 def test_matvec_wide_rows(wtype, rows, cols, epilogue):
     """The any-width kernel where its division of the rows changes: one row, an odd last row, widths that end inside a
-    line, waves without rows, waves with as many rows as they take (600000 rows).  The error against 64 bits stays
+    line, waves without rows, waves with as many rows as they take (600000 rows); and both sides of the row counts at
+    which the choice of kernel or of rows per wave changes.  The error against 64 bits stays
     under cols roundings of 2^-24 of the inputs, in the root mean square about sqrt(cols) of them: 1e-5 is ten times."""
     import torch
     g = torch.Generator(device="cuda")
