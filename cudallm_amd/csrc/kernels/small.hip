@@ -32,19 +32,23 @@ int device_cu_count() {
 // kDefaultRpb is the rpb used when the caller passes 0.  kGridPerCu caps the grid at that many workgroups per CU
 // (0: as many as can be resident at once).  Smaller grids mean fewer workgroups, each with more passes, so fewer
 // repeats of the input and norm prologue; larger ones than can be resident spread the last passes more evenly over
-// many rows.  Measured effects: bf16 qkv 4.69 -> 4.40 us, gate_up 12.50 -> 12.00, down 7.65 -> 7.50, lm_head
-// 79.8 -> 78.0 (8 per CU) -> 77.0 (16); int8 gate_up 8.53 -> 7.25, down 5.94 -> 5.77 (rpb 4 -> 2, 2 per CU), lm_head
-// 43.6 -> 42.0 (8 per CU), 20483 x 2048 9.05 -> 8.76 (2 per CU); int4 gate_up 7.72 -> 6.68, lm_head 24.3 -> 23.4
-// (2 -> 8 per CU), 20483 x 2048 6.67 -> 6.04 (2 per CU).
+// many rows, and the prologue of one workgroup runs under the loads of the others.  Measured, us:
+//   bf16  qkv 4.69 -> 4.40, gate_up 12.50 -> 12.00 (1 per CU); 8192 columns 7.65 -> 7.50;
+//         128256 x 2048 81.7 (8 per CU) / 81.3 (16) / 80.0 (32) / 75.3 to 77.9 (one row block each); 256000 rows 158
+//         (16) / 146 to 152, 100000 rows 63.8 / 61.6
+//   int8  gate_up 8.53 -> 7.25 (1 per CU), down 5.94 -> 5.77 (rpb 4 -> 2, 2 per CU), 20483 x 2048 9.05 -> 8.76 (2 per CU);
+//         128256 x 2048 42.8 (8 per CU) / 41.6 (64), 256000 rows 80.9 / 78.7, 100000 rows 34.2 / 33.6
+//   int4  gate_up 7.72 -> 6.68 (1 per CU), 20483 x 2048 6.67 -> 6.04 (2 per CU); 128256 x 2048 24.3 (2 per CU) /
+//         23.6 (8) / 24.7 (16)
 constexpr int kDefaultRpb[3][4] = {
     {1, 1, 2, 2},  // bf16
     {4, 2, 2, 4},  // int8
     {4, 4, 4, 4},  // int4
 };
 constexpr int kGridPerCu[3][4] = {
-    {1, 1, 2, 16},  // bf16
-    {2, 1, 2, 8},   // int8
-    {2, 1, 2, 8},   // int4
+    {1, 1, 2, 1024},  // bf16: one row block per workgroup, up to 2 M rows
+    {2, 1, 2, 64},    // int8
+    {2, 1, 2, 8},     // int4
 };
 
 namespace {
