@@ -565,8 +565,7 @@ void launch_attention_splitk_static(const float* q, const uint16_t* k_cache, con
     CLLM_REQUIRE(static_cast<long long>(nh) * (max_seq / kAttnChunk) <= kStaticAttnSlots,
                  "attention (static scratch): nh * max_seq / 128 exceeds the 8192 partial slots of the static scratch");
     float* base = scratch_on_current_device();
-    // No clearing needed: every split at or before ctx writes its slots before the merge reads them, and the merge
-    // reads no other slot.
+    // No clearing needed: a partial's words carry their launch's number, and the merge takes only words of its own launch.
     launch_attention_splitk(q, k_cache, v_cache, d_pos, base, base + static_cast<size_t>(kStaticAttnSlots) * kHd, out,
                             nh, nkv, hd, max_seq, s);
 }

@@ -82,20 +82,6 @@ __device__ __forceinline__ float sum_lanes_xor(float x) {
     return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
 }
 
-// The permlane swap itself on two values: afterwards a + b is, in lanes with bit M clear, a's sum over the pair
-// (l, l ^ M) and, in lanes with it set, b's sum (each pair of values is folded into one, with no selects).
-template <int M>
-__device__ __forceinline__ float fold_lanes(float x, float y) {
-    static_assert(M == 16 || M == 32, "row swaps");
-    unsigned a = __builtin_bit_cast(unsigned, x), b = __builtin_bit_cast(unsigned, y);
-    if constexpr (M == 16) {
-        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-    } else {
-        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-    }
-    return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
-}
-
 // max of x over lanes l and l ^ M, for M = 16 or 32.
 template <int M>
 __device__ __forceinline__ float max_lanes_xor(float x) {
