@@ -13,8 +13,8 @@
 //  * R rows (rpb) are loaded before any is consumed, for R x (4 KiB bf16 | 2 KiB int8 | 1 KiB int4)
 //    of loads per pass; a wave issues the next pass's loads before it multiplies the current one,
 //    so up to 2R rows are in flight.  The first pass's weights are requested right after the lane's
-//    inputs, before the norm and digit prologue.  No load sits under a branch (rows past the end
-//    re-read the last row) and, with KS = 1, no store sits in the loop (each wave's row sums wait in
+//    inputs, before the norm and digit prologue, and with them, for some quantised forms, what is read
+//    beside the sums at the end.  No load sits under a branch (rows past the end re-read the last row) and, with KS = 1, no store sits in the loop (each wave's row sums wait in
 //    its lanes until its last pass): either made the compiler's wait counts conservative, so that a
 //    pass also waited for the next pass's loads (128256 x 2048, bf16 82.5 -> 80.0 us, int8 44.6 -> 40.5,
 //    int4 32.2 -> 28.0).  With the launches of small.hip the same shape now takes 77.9, 41.4 and 23.7 us on
@@ -89,6 +89,14 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     constexpr bool GLU = EP == Epilogue::SWIGLU;
     constexpr int NP = GLU ? 2 : 1;
     constexpr bool DIG = WT != WType::BF16 && KS == 1;
+    // Quantised 8192-wide rows: what the merge of the slices reads (old outputs, int8's scales) comes with the pass's
+    // weights instead of after its sums.  20000 rows int8 30.7 -> 27.9 us, int4 22.4 -> 20.9; 2048 rows 5.73 -> 5.59, 5.20 ->
+    // 5.10.  bf16, where a pass is twice the bytes, gains nothing (20000 rows 52.6 -> 53.2) and reads them in the merge.
+    constexpr bool EARLY = KS > 1 && WT != WType::BF16;
+    // Likewise the rows' sums of quantised ADD with KS = 1, once for all passes: 512 rows int8 2.86 -> 2.58 us, int4 2.94 ->
+    // 2.67; 2048 rows 3.20 -> 3.15, 3.08 -> 2.92; 20483 rows 8.81 -> 8.68, 6.22 -> 6.10.  Not int8's scales of STORE (3072 rows
+    // 3.24 against 3.27) and SWIGLU (16384 rows 7.48 against 7.66), nor bf16 (512 rows 2.75 against 3.02).
+    constexpr bool EARLY_SUM = KS == 1 && WT != WType::BF16 && EP == Epilogue::ADD;
     // x^ by lines of 64 chunks, a lane's 16-byte words of a line at [line][word][lane]: the digits of a chunk, or its
     // floats.  One copy with KS = 1, a slice per wave with KS > 1.
     constexpr int XW = !DIG ? F::CPC / 4 : WT == WType::INT4 ? 6 : 3;
@@ -139,6 +147,7 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
         u32x4 v[R][F::CPL];
         u32x4 vu[GLU ? R : 1][F::CPL];
         uint16_t g[R], gu[R];
+        float y, sc, scu;  // EARLY: of the thread's row in the merge
     };
     // Rows past the end load the last row again (their sums are never stored): with no branch around the loads the
     // compiler counts them exactly, so a pass waits only for its own loads and not for the next pass's as well.
@@ -158,9 +167,23 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
                 if constexpr (GLU) b.gu[i] = gload(sbase + static_cast<size_t>(rc + out_rows) * groups_per_row + soff);
             }
         }
+        if constexpr (EARLY) {
+            const int rc = min(r0 - grp * R + min(tid, ROWS_WG - 1), out_rows - 1);
+            if constexpr (EP == Epilogue::ADD) b.y = a.y[rc];
+            if constexpr (WT == WType::INT8) {
+                b.sc = static_cast<const float*>(a.scales)[rc];
+                if constexpr (GLU) b.scu = static_cast<const float*>(a.scales)[rc + out_rows];
+            }
+        }
     };
     Block A, B;
     load(A, base + grp * R);
+    [[maybe_unused]] float old_y = 0.f, sum_scale = 1.f;
+    if constexpr (EARLY_SUM) {  // the row that lane l keeps to the end
+        const int rc = min(base + min(lane / R, left - 1) * stride + grp * R + lane % R, out_rows - 1);
+        old_y = a.y[rc];
+        if constexpr (WT == WType::INT8) sum_scale = static_cast<const float*>(a.scales)[rc];
+    }
     __builtin_amdgcn_sched_barrier(0);  // keep the weight loads ahead of the prologue
 
     // RMSNorm's sum of squares and, for the digits, the largest |x norm_w| (infinite if any input is infinite or NaN).
@@ -364,11 +387,14 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
                     if constexpr (GLU) su += part[(q * ROWS_WG + tid) * NP + 1];
                 }
                 if constexpr (WT == WType::INT8) {
-                    const float* sc = static_cast<const float*>(a.scales);
-                    s *= sc[r];
-                    if constexpr (GLU) su *= sc[r + out_rows];
+                    s *= b.sc;
+                    if constexpr (GLU) su *= b.scu;
                 }
-                store_out<EP>(a.y, r, s, su);
+                if constexpr (EARLY && EP == Epilogue::ADD) {
+                    a.y[r] = b.y + s;
+                } else {
+                    store_out<EP>(a.y, r, s, su);
+                }
             }
             __syncthreads();
         }
@@ -398,12 +424,16 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     }
     if constexpr (KS == 1) {
         if (lane < held && acc_row < out_rows) {
-            if constexpr (WT == WType::INT8) {
-                const float* sc = static_cast<const float*>(a.scales);
-                acc *= sc[acc_row];
-                if constexpr (GLU) acc_u *= sc[acc_row + out_rows];
+            if constexpr (EARLY_SUM) {
+                a.y[acc_row] = old_y + acc * sum_scale;
+            } else {
+                if constexpr (WT == WType::INT8) {
+                    const float* sc = static_cast<const float*>(a.scales);
+                    acc *= sc[acc_row];
+                    if constexpr (GLU) acc_u *= sc[acc_row + out_rows];
+                }
+                store_out<EP>(a.y, acc_row, acc, acc_u);
             }
-            store_out<EP>(a.y, acc_row, acc, acc_u);
         }
     }
 }
