@@ -60,9 +60,14 @@ __device__ __forceinline__ void store_out(float* y, int r, float d, float du) {
     }
 }
 
-// The fixed-point scale of the digits here fills the digits' whole range (|xi| up to about 2^23, a bit more than digits.h's
-// own words hold), so that the rounding of x^ adds no more than the sums in 32 bits did: 24576 x 4096 int4 with SWIGLU,
-// against 64 bits: 5.1e-7 converting every weight, 8.1e-7 with |xi| < 2^22, 4.2e-7 so.
+// The fixed-point scale of the digits here fills the digits' whole range (|xi| up to about 2^23, a bit more than the decode
+// kernel's words of digits.h hold).  An input is rounded by up to 2^-24 .. 2^-23 of the largest |x^| that shares its scale,
+// so how many share one matters once inputs differ in size.  matvec_fast has one scale for the 2048 columns of a row,
+// matvec_wide one per chunk (16 columns of int8, 32 of int4).  Errors against 64 bits, root mean square over 12 seeds, of 8192
+// x 4096 int4 with norm and SWIGLU and of 4096 x 12288 int8, with x^ in floats and every weight converted / one scale
+// per row / one per chunk: normal inputs 9.4e-7 / 4.2e-7 / 2.7e-7 and 4.0e-7 / 2.5e-7 / 1.6e-7; one input 1000 to 2000
+// times the rest 8.8e-7 / 5.3e-6 / 5.1e-7 and 3.9e-7 / 5.3e-6 / 2.1e-7; the same meeting zero weights (where the floats
+// lose the bits of its chunk to the bias of the converted weights) 2.0e-5 / 1.2e-4 / 1.0e-5 and 4.8e-6 / 7.1e-5 / 2.5e-6.
 template <WType WT>
 __device__ __forceinline__ int wide_exponent(float m) {
     if (!(m > 0.f) || !(m < INFINITY)) return 0;
@@ -443,8 +448,10 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
 // Bound by the weight bytes (int4 by instruction issue beside them).  x^ is staged in LDS once per workgroup in the order
 // in which the lanes of a wave read it, so a wave takes whole rows of any width: a step is one 1 KiB line (64 chunks) of
 // two rows, the gate and the up row with SWIGLU, else two neighbours, which share the LDS reads of x^.  The quantised
-// types stage x^ as the digit words of digits.h (a line's digit d of lane l at [line][d][l], 16 bytes; a third to a half
-// of the instructions of converting every weight), bf16 as float4s ([line][quad][l]).  The steps of all of a wave's rows
+// types stage x^ as digit words (a line's digit d of lane l at [line][d][l], 16 bytes; a third to a half of the
+// instructions of converting every weight) with a scale of its own for every lane's chunk (one scale for the row measured
+// no faster: 24576 x 4096 int4 11.5 us both, 4096 x 12288 int4 8.6 against 8.5, int8 11.6 against 11.3), bf16 as float4s
+// ([line][quad][l]).  The steps of all of a wave's rows
 // are one sequence with kDepth steps in flight; the loads are buffer loads, so the ones past the wave's last row and past
 // a row's end (widths that are not a whole number of lines) return 0 without a memory access and no load sits under a
 // branch.  Row sums wait in LDS for the wave's end, so no store sits in the loop either.
@@ -462,9 +469,10 @@ struct Wide {
     using F = Fmt<WT>;
     static constexpr int Q = WT == WType::INT4 ? 6 : WT == WType::INT8 ? 3 : 2;  // 16-byte words of x^ per chunk
     static __host__ __device__ int lines(int cols) { return (cols / F::CPC + kWave - 1) / kWave; }
-    // x^, then the row sums.
+    // x^, the chunks' scales (quantised types), then the row sums.
     static size_t smem(int cols, int units_per_wave) {
-        return static_cast<size_t>(lines(cols)) * kWave * Q * 16 + sizeof(float) * kWideWaves * 2 * units_per_wave;
+        return static_cast<size_t>(lines(cols)) * kWave * (Q * 16 + (WT != WType::BF16 ? 4 : 0)) +
+               sizeof(float) * kWideWaves * 2 * units_per_wave;
     }
 };
 
@@ -474,10 +482,11 @@ __global__ void __launch_bounds__(kWideThreads) matvec_wide(MatvecArgs a, int un
     constexpr bool GLU = EP == Epilogue::SWIGLU, DIG = WT != WType::BF16;
     constexpr int Q = Wide<WT>::Q;
     extern __shared__ u32x4 xs[];  // [line][Q][lane]
-    __shared__ float sred[kWideWaves], mred[kWideWaves];
+    __shared__ float sred[kWideWaves];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
     const int nchunk = a.cols / F::CPC, nk = Wide<WT>::lines(a.cols), rem = nchunk - (nk - 1) * kWave;
-    float* const sums = reinterpret_cast<float*>(xs + nk * Q * kWave) + wave * 2 * max_units;
+    float* const chunk_scale = reinterpret_cast<float*>(xs + nk * Q * kWave);  // DIG: [line][lane]
+    float* const sums = chunk_scale + (DIG ? nk * kWave : 0) + wave * 2 * max_units;
 
     // Units [u0, u0 + n) of this wave.
     const int64_t wi = blockIdx.x * kWideWaves + wave, nw = gridDim.x * kWideWaves;
@@ -543,34 +552,20 @@ __global__ void __launch_bounds__(kWideThreads) matvec_wide(MatvecArgs a, int un
     for (int d = 0; d < kDepth<WT>; ++d) load(st[d]);
     __builtin_amdgcn_sched_barrier(0);
 
-    // The sum of squares (norm) and the largest |x norm_w| (digits; infinite if any input is infinite or NaN).
-    [[maybe_unused]] float inv = 1.f, dsc = 1.f, scale = 1.f;
-    if constexpr (NORM || DIG) {
-        float ss = 0.f, mx = 0.f;
+    [[maybe_unused]] float inv = 1.f;
+    if constexpr (NORM) {
+        float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < kXPairs; ++i)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float v = xv[i][e / 4][e % 4];
-                ss = fmaf(v, v, ss);
-                if constexpr (DIG) {
-                    const float t = NORM ? v * nv[i][e / 4][e % 4] : v;
-                    mx = fabsf(t) < INFINITY ? fmaxf(mx, fabsf(t)) : INFINITY;
-                }
-            }
-        if constexpr (NORM) ss = wave_sum(ss);
-        if constexpr (DIG) mx = wave_max(mx);
-        if (lane == 0) sred[wave] = ss, mred[wave] = mx;
+            for (int e = 0; e < 8; ++e) ss = fmaf(xv[i][e / 4][e % 4], xv[i][e / 4][e % 4], ss);
+        ss = wave_sum(ss);
+        if (lane == 0) sred[wave] = ss;
         __syncthreads();
-        ss = 0.f, mx = 0.f;
+        ss = 0.f;
 #pragma unroll
-        for (int w = 0; w < kWideWaves; ++w) ss += sred[w], mx = fmaxf(mx, mred[w]);
-        if constexpr (NORM) inv = rsqrtf(ss / static_cast<float>(a.cols) + a.eps);
-        if constexpr (DIG) {
-            const int e = wide_exponent<WT>(mx * inv);
-            scale = ldexpf(1.f, e);
-            dsc = mx * inv < INFINITY ? ldexpf(1.f, -e) : __builtin_nanf("");
-        }
+        for (int w = 0; w < kWideWaves; ++w) ss += sred[w];
+        inv = rsqrtf(ss / static_cast<float>(a.cols) + a.eps);
     }
 #pragma unroll
     for (int i = 0; i < kXPairs; ++i) {
@@ -584,6 +579,18 @@ __global__ void __launch_bounds__(kWideThreads) matvec_wide(MatvecArgs a, int un
             if constexpr (NORM) v[e] = v[e] * inv * nv[i][e / 4][e % 4];
         }
         uint32_t* const xw = reinterpret_cast<uint32_t*>(xs);
+        // The chunk's scale from its largest |x^| (infinite if one of them is infinite or NaN: its dots are NaN then).
+        [[maybe_unused]] float scale = 1.f;
+        if constexpr (DIG) {
+            float m = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) m = fabsf(v[e]) < INFINITY ? fmaxf(m, fabsf(v[e])) : INFINITY;
+            m = fmaxf(m, dpp<kDppXor1>(m));
+            if constexpr (F::CPC == 32) m = fmaxf(m, dpp<kDppXor2>(m));
+            const int e = wide_exponent<WT>(m);
+            scale = ldexpf(1.f, e);
+            if (j % (F::CPC / 8) == 0) chunk_scale[j / (F::CPC / 8)] = m < INFINITY ? ldexpf(1.f, -e) : __builtin_nanf("");
+        }
         if constexpr (WT == WType::BF16) {
 #pragma unroll
             for (int q = 0; q < 2; ++q)
@@ -611,14 +618,15 @@ __global__ void __launch_bounds__(kWideThreads) matvec_wide(MatvecArgs a, int un
     }
     __syncthreads();
 
-    // Row sums: float for bf16 and int4 (per line, times the group scale), exact integers per digit for int8.
+    // Row sums: floats, a line's exact integer dots times the chunk's scale (and int4's group scale) added line by line.
     float acc[2] = {0.f, 0.f};
-    [[maybe_unused]] int ia[2][3] = {{0, 0, 0}, {0, 0, 0}};
     int k = 0, u = 0;
     auto step = [&](const Step& b) {
         u32x4 x[Q];
 #pragma unroll
         for (int q = 0; q < Q; ++q) x[q] = xs[(k * Q + q) * kWave + lane];
+        [[maybe_unused]] float xscale = 1.f;
+        if constexpr (DIG) xscale = chunk_scale[k * kWave + lane];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             if constexpr (WT == WType::BF16) {
@@ -627,11 +635,14 @@ __global__ void __launch_bounds__(kWideThreads) matvec_wide(MatvecArgs a, int un
                 for (int e = 0; e < 8; ++e) xf[e] = __builtin_bit_cast(f32x4, x[e / 4])[e % 4];
                 acc[i] += chunk_dot<WT>(b.v[i], xf);
             } else if constexpr (WT == WType::INT8) {
+                int c[3] = {0, 0, 0};
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
 #pragma unroll
                     for (int d = 0; d < 3; ++d)
-                        ia[i][d] = __builtin_amdgcn_sdot4(static_cast<int>(b.v[i][t]), static_cast<int>(x[d][t]), ia[i][d], false);
+                        c[d] = __builtin_amdgcn_sdot4(static_cast<int>(b.v[i][t]), static_cast<int>(x[d][t]), c[d], false);
+                // c[0] + 256 c[1] stays below 2^27.
+                acc[i] = fmaf(fmaf(static_cast<float>(c[2]), 65536.f, static_cast<float>(c[0] + 256 * c[1])), xscale, acc[i]);
             } else {
                 int c[6] = {0, 0, 0, 0, 0, 0};
 #pragma unroll
@@ -641,16 +652,11 @@ __global__ void __launch_bounds__(kWideThreads) matvec_wide(MatvecArgs a, int un
                     for (int d = 0; d < 6; ++d) c[d] = __builtin_amdgcn_sdot8(w, static_cast<int>(x[d][t]), c[d], false);
                 }
                 const int p0 = c[0] + 16 * c[1], p1 = c[2] + 16 * c[3], p2 = c[4] + 16 * c[5];
-                acc[i] = fmaf(fmaf(static_cast<float>(p2), 65536.f, static_cast<float>(p0 + 256 * p1)), half_bits_to_float(b.g[i]), acc[i]);
+                const float p = fmaf(static_cast<float>(p2), 65536.f, static_cast<float>(p0 + 256 * p1));
+                acc[i] = fmaf(p * xscale, half_bits_to_float(b.g[i]), acc[i]);
             }
         }
         if (++k == nk) {
-            if constexpr (WT == WType::INT8)
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    acc[i] = fmaf(fmaf(static_cast<float>(ia[i][2]), 256.f, static_cast<float>(ia[i][1])), 256.f, static_cast<float>(ia[i][0]));
-                    ia[i][0] = ia[i][1] = ia[i][2] = 0;
-                }
             const float t = rows_sum<2>(acc, lane);
             if (lane < 2) sums[2 * u + lane] = t;
             acc[0] = acc[1] = 0.f;
@@ -671,7 +677,7 @@ __global__ void __launch_bounds__(kWideThreads) matvec_wide(MatvecArgs a, int un
     for (int i = lane; i < (GLU ? n : 2 * n); i += kWave) {
         const int r = r0 + i;
         if (r >= out_rows) break;
-        float d = sums[GLU ? 2 * i : i] * dsc, du = GLU ? sums[2 * i + 1] * dsc : 0.f;
+        float d = sums[GLU ? 2 * i : i], du = GLU ? sums[2 * i + 1] : 0.f;
         if constexpr (WT == WType::INT8) {
             const float* sc = static_cast<const float*>(a.scales);
             d *= sc[r];
@@ -742,9 +748,11 @@ template <WType WT, Epilogue EP, bool NORM>
 void pick_shape(int rpb, const MatvecArgs& a, hipStream_t s) {
     if (a.cols == 2048) return pick_r<WT, EP, NORM, 1>(rpb, a, s);
     // Quantised 8192-wide rows convert every weight in matvec_fast, for want of columns per wave to share the digits of
-    // x^ with; with two matrices of many rows the any-width kernel's digits are faster: SWIGLU rows 4096 / 8192 / 30000, int4
-    // 8.8 / 13.2 / 38.9 -> 7.7 / 11.0 / 25.6 us, int8 9.3 / 15.6 / 47.7 -> 9.2 / 14.5 / 45.3.  Without SWIGLU matvec_fast
-    // stays ahead at most row counts (2048: int4 5.1 against 6.2, int8 5.7 against 6.6; 16384: int8 26.2 against 27.1).
+    // x^ with; with two matrices of many rows the any-width kernel's digits are faster for int4: SWIGLU without norm, rows
+    // 4096 / 8192 / 30000, 7.3 / 11.9 / 36.0 -> 6.5 / 9.5 / 23.9 us.  int8 is no faster (7.9 / 13.4 / 39.4 against 8.1 /
+    // 13.0 / 41.9; 6000 rows 10.8 against 12.1) but has a third of the error against 64 bits (8.0e-7 -> 2.5e-7).
+    // Without SWIGLU matvec_fast stays ahead at most row counts (ADD, 2048 / 8192 / 16384 / 30000 rows: int8 5.6 / 12.9 /
+    // 22.9 / 37.8 against 6.3 / 13.2 / 25.4 / 39.6, int4 4.9 / 9.9 / 16.4 / 27.0 against 5.8 / 10.3 / 15.7 / 24.0).
     if (a.cols == 8192 && !(WT != WType::BF16 && EP == Epilogue::SWIGLU && a.rows >= 4096)) return pick_r<WT, EP, NORM, 4>(rpb, a, s);
     return launch_wide<WT, EP, NORM>(a, s);
 }

@@ -163,6 +163,56 @@ def test_matvec_wide_non_finite_input(wtype, norm, value):
         assert np.isnan(y).all()
 
 
+@pytest.mark.parametrize("wtype", ["int8", "int4"])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("outlier", [1e3, 1e6])
+@pytest.mark.parametrize("rows,cols,epilogue", [(1001, 1024, "store"), (500, 5120, "add"), (300, 12288, "store"),
+                                                (4096, 8192, "swiglu")])
+def test_matvec_wide_outlier_input(wtype, norm, outlier, rows, cols, epilogue):
+    """One input far above the others that meets zero weights: it may cost the 16 (int8) or 32 (int4) inputs of its own
+    chunk bits, and no others.  A chunk's fixed-point words have a step of at most 2 m / 7829350 for its largest input m,
+    which leaves a row an error of sigma = that step / sqrt(12) times the 2-norm of the row's weights in the chunk.  Bound
+    for every row: 8 sigma, and 1e-6 (16 roundings) of the 2-norms of the row and of the other inputs.  One scale for all
+    columns leaves 8 (1024 columns) to 28 sigma in the root mean square over the rows, and more than three times that in
+    the worst of them."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows + cols)
+    n, col, chunk = rows // 2 if epilogue == "swiglu" else rows, cols // 2 + 37, 32 if wtype == "int4" else 16
+    top = 7 if wtype == "int4" else 127
+    q = torch.randint(-top, top + 1, (rows, cols), generator=g, device="cuda", dtype=torch.int8)
+    q[:, col] = 0
+    if wtype == "int8":
+        w, scales = q, torch.ones(rows, device="cuda")
+    else:
+        u = (q + 8).view(rows, cols // 2, 2).to(torch.uint8)
+        w, scales = u[..., 0] | (u[..., 1] << 4), torch.ones(rows, cols // 128, device="cuda").half()
+    x, nw = torch.randn(cols, generator=g, device="cuda"), torch.rand(cols, generator=g, device="cuda") + 0.5
+    x[col] = outlier
+    y0 = torch.randn(n, generator=g, device="cuda")
+    y = y0.clone()
+    E.launch_matvec(wtype, epilogue, 0, w.data_ptr(), scales.data_ptr(), x.data_ptr(), nw.data_ptr() if norm else None, 1e-5,
+                    y.data_ptr(), rows, cols, torch.cuda.current_stream().cuda_stream)
+    xn = x.double()
+    if norm:
+        xn = xn * torch.rsqrt((xn * xn).mean() + 1e-5) * nw.double()
+    m = q.double()
+    d = m @ xn
+    c0 = col // chunk * chunk
+    sigma = 2 * xn[col].abs() / 7829350 / 12 ** 0.5 * m[:, c0:c0 + chunk].norm(dim=1)
+    rest = xn.clone()
+    rest[col] = 0.0
+    bound = 8 * sigma + 1e-6 * m.norm(dim=1) * rest.norm()
+    if epilogue == "swiglu":  # silu's slope is at most 1.1
+        act = torch.nn.functional.silu(d[:n])
+        ref, bound = act * d[n:], 1.1 * bound[:n] * (d[n:].abs() + bound[n:]) + act.abs() * bound[n:] + 1e-6 * (act * d[n:]).abs()
+    else:
+        ref = d + y0.double() if epilogue == "add" else d
+        bound = bound + 1e-6 * ref.abs()
+    excess = ((y.double() - ref).abs() / bound).max().item()
+    assert excess <= 1, f"{excess} times the bound"
+
+
 def test_stream_read_timed_hook():
     """The bandwidth kernel on a device buffer through its timed hook: every launch shape records both events, and the
     sink (written only for one XOR-folded word that a zero buffer never gives) stays untouched."""
