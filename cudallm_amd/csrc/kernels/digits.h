@@ -1,9 +1,12 @@
-// Fixed-point digits of a normalised input for the integer dot products of the quantised weights, shared by the
-// persistent decode kernel and the standalone matvec.  The input x^ is written as a 22-bit fixed-point integer with
-// one power-of-two scale, xi = rint(x^ 2^e) (|xi| <= 2^22), offset by C so that every base-256 (int8) or base-16
-// (int4) digit is non-negative, and packed in the weights' own layout; xor C then makes each digit signed, so that
-// v_dot4_i32_i8 / v_dot8_i32_i4 multiply raw weight words by digits.  The integer sums are exact; the only new
-// rounding is that of xi (at most 2^-23 of max |x^|), against fp32's 2^-24 of each |x^|.
+// Fixed-point digits of a normalised input for the integer dot products of the quantised weights.  The input x^ is
+// written as a fixed-point integer with a power-of-two scale, xi = rint(x^ 2^e), offset by C so that every base-256
+// (int8) or base-16 (int4) digit is non-negative, and packed in the weights' own layout; xor C then makes each digit
+// signed, so that v_dot4_i32_i8 / v_dot8_i32_i4 multiply raw weight words by digits.  The integer sums are exact; the
+// only new rounding is that of xi, against fp32's 2^-24 of each |x^|.
+//  * The persistent decode kernel: |xi| <= 2^22 with one scale per vector (dig_exponent, fixed_word), rounded by at
+//    most 2^-23 of max |x^|.
+//  * The standalone matvec packs its words here too, with wider ones (|xi| up to about 2^23) and a scale for every 16
+//    or 32 columns (wide_exponent and wide_word in matvec_impl.h).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -12,7 +15,7 @@
 
 namespace cllm {
 
-// Exponent e of the fixed-point scale from a bound m >= max |x^|: m 2^e < 2^22.  At most 126, so that 2^e and 2^-e
+// Exponent e of the decode kernel's fixed-point scale from a bound m >= max |x^|: m 2^e < 2^22.  At most 126, so that 2^e and 2^-e
 // are normal floats (inputs below 2^-104 then keep fewer bits, which changes nothing measurable).
 __device__ __forceinline__ int dig_exponent(float m) {
     if (!(m > 0.f) || !(m < INFINITY)) return 0;

@@ -14,14 +14,17 @@
 //    of loads per pass; a wave issues the next pass's loads before it multiplies the current one,
 //    so up to 2R rows are in flight.  The first pass's weights are requested right after the lane's
 //    inputs, before the norm and digit prologue, and with them, for some quantised forms, what is read
-//    beside the sums at the end.  No load sits under a branch (rows past the end re-read the last row) and, with KS = 1, no store sits in the loop (each wave's row sums wait in
-//    its lanes until its last pass): either made the compiler's wait counts conservative, so that a
-//    pass also waited for the next pass's loads (128256 x 2048, bf16 82.5 -> 80.0 us, int8 44.6 -> 40.5,
+//    beside the sums at the end.  No load sits under a branch (rows past the end re-read the last row)
+//    and, with KS = 1, no store sits in the loop (each wave's row sums wait in its lanes until its last
+//    pass): either made the compiler's wait counts conservative, so that a pass also waited for the next
+//    pass's loads (128256 x 2048, bf16 82.5 -> 80.0 us, int8 44.6 -> 40.5,
 //    int4 32.2 -> 28.0).  With the launches of small.hip the same shape now takes 77.9, 41.4 and 23.7 us on
 //    MI355X: 6.7, 6.3 and 5.7 TB/s, where a plain stream read reaches 7.1.
 //  * Quantised 2048-wide rows (KS = 1) use integer digit dots: the workgroup turns the inputs into
-//    fixed-point digit words once (one scale from max |x^|), and a row then costs 24 v_dot8_i32_i4 / v_dot4_i32_i8 per lane instead of
-//    a conversion and an FMA per column.  The 8192-wide down rows (KS = 4) keep the float path.
+//    fixed-point digit words once (with a scale for each 16-byte chunk's columns), and a row then costs
+//    24 v_dot8_i32_i4 / v_dot4_i32_i8 per lane instead of a conversion and an FMA per column.  A scale per chunk
+//    instead of one per row costs up to 2 % (128256 x 2048 int4 22.8 -> 23.2 us, int8 39.3 -> 39.5; 3072 x 2048
+//    2.82 -> 2.83 and 3.21 -> 3.26; 16384 x 2048 SWIGLU 5.23 -> 5.23 and 7.44 -> 7.49).  The 8192-wide down rows (KS = 4) keep the float path.
 //  * Row sums are wave64 DPP butterflies (deterministic order); with KS > 1 the slice partials
 //    meet in LDS and are added in slice order.  No atomics anywhere.
 //  * The grid: min(row blocks, CUs x the shape class's workgroups per CU (grid_per_cu; by default as
@@ -61,13 +64,15 @@ __device__ __forceinline__ void store_out(float* y, int r, float d, float du) {
 }
 
 // The fixed-point scale of the digits here fills the digits' whole range (|xi| up to about 2^23, a bit more than the decode
-// kernel's words of digits.h hold).  An input is rounded by up to 2^-24 .. 2^-23 of the largest |x^| that shares its scale,
-// so how many share one matters once inputs differ in size.  matvec_fast has one scale for the 2048 columns of a row,
-// matvec_wide one per chunk (16 columns of int8, 32 of int4).  Errors against 64 bits, root mean square over 12 seeds, of 8192
-// x 4096 int4 with norm and SWIGLU and of 4096 x 12288 int8, with x^ in floats and every weight converted / one scale
-// per row / one per chunk: normal inputs 9.4e-7 / 4.2e-7 / 2.7e-7 and 4.0e-7 / 2.5e-7 / 1.6e-7; one input 1000 to 2000
-// times the rest 8.8e-7 / 5.3e-6 / 5.1e-7 and 3.9e-7 / 5.3e-6 / 2.1e-7; the same meeting zero weights (where the floats
-// lose the bits of its chunk to the bias of the converted weights) 2.0e-5 / 1.2e-4 / 1.0e-5 and 4.8e-6 / 7.1e-5 / 2.5e-6.
+// kernel's words of digits.h hold).  An input is rounded by up to 2^-24 .. 2^-23 of the largest |x^| that shares its scale:
+// those of one chunk, 16 columns of int8 or 32 of int4.  Errors against 64 bits, root mean square over 12 seeds, with x^ in
+// floats and every weight converted / with one scale for a whole row / with one per chunk:
+//                                   normal inputs              one 1000 to 2000 times the rest  it meets zero weights
+//   int4  8192 x 4096 norm, SWIGLU  9.4e-7 / 4.2e-7 / 2.7e-7   8.8e-7 / 5.3e-6 / 5.1e-7         2.0e-5 / 1.2e-4 / 1.0e-5
+//   int8  4096 x 12288              4.0e-7 / 2.5e-7 / 1.6e-7   3.9e-7 / 5.3e-6 / 2.1e-7         4.8e-6 / 7.1e-5 / 2.5e-6
+//   int4  3072 x 2048 norm                 - / 2.8e-7 / 1.7e-7        - / 2.5e-6 / 3.2e-7              - / 7.8e-5 / 9.3e-6
+// (The floats lose the bits of the large input's chunk to the bias of the converted weights.)  A scale per row also needed
+// the largest |x norm_w| before the norm was known, which is infinite for products past the floats whose x^ are not.
 template <WType WT>
 __device__ __forceinline__ int wide_exponent(float m) {
     if (!(m > 0.f) || !(m < INFINITY)) return 0;
@@ -77,6 +82,21 @@ __device__ __forceinline__ int wide_exponent(float m) {
 }
 __device__ __forceinline__ uint32_t wide_word(float v, float scale, uint32_t C) {
     return static_cast<uint32_t>(static_cast<int>(rintf(v * scale))) + C;
+}
+
+// A thread has 8 neighbouring x^ (thread j columns 8 j ..): the scale of its chunk's fixed-point words, from the chunk's
+// largest |x^|; the inverse goes to chunk_scale[chunk] (NaN if one of them is infinite or NaN: the chunk's dots then are).
+template <WType WT>
+__device__ __forceinline__ float set_chunk_scale(const float* v, int j, float* chunk_scale) {
+    constexpr int THREADS = Fmt<WT>::CPC / 8;  // per chunk, neighbours
+    float m = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m = fabsf(v[e]) < INFINITY ? fmaxf(m, fabsf(v[e])) : INFINITY;
+    m = fmaxf(m, dpp<kDppXor1>(m));
+    if constexpr (THREADS == 4) m = fmaxf(m, dpp<kDppXor2>(m));
+    const int e = wide_exponent<WT>(m);
+    if (j % THREADS == 0) chunk_scale[j / THREADS] = m < INFINITY ? ldexpf(1.f, -e) : __builtin_nanf("");
+    return ldexpf(1.f, e);
 }
 
 typedef __amdgpu_buffer_rsrc_t Rsrc;
@@ -106,7 +126,8 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     // floats.  One copy with KS = 1, a slice per wave with KS > 1.
     constexpr int XW = !DIG ? F::CPC / 4 : WT == WType::INT4 ? 6 : 3;
     __shared__ u32x4 xs[KS][F::CPL * XW * kWave];
-    __shared__ float scratch[16];
+    __shared__ float chunk_scale[DIG ? kSlice / F::CPC : 1];
+    __shared__ float scratch[4];
     __shared__ float part[KS > 1 ? KS * ROWS_WG * NP : 1];
 
     const int tid = threadIdx.x;
@@ -116,7 +137,7 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     const int slice = wave % KS, grp = wave / KS;
     const int out_rows = GLU ? a.rows / 2 : a.rows;
     // Row blocks are dealt to the workgroups in turn; base is the same for every wave of a workgroup, so the
-    // barriers below (block_sum, and pass() with KS > 1) are reached by all of them.
+    // barriers below (the prologue's, and pass()'s with KS > 1) are reached by all of them.
     const int stride = gridDim.x * ROWS_WG;
     int base = blockIdx.x * ROWS_WG;
     if (base >= out_rows) return;
@@ -191,44 +212,27 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     }
     __builtin_amdgcn_sched_barrier(0);  // keep the weight loads ahead of the prologue
 
-    // RMSNorm's sum of squares and, for the digits, the largest |x norm_w| (infinite if any input is infinite or NaN).
-    float inv = 1.f;
-    [[maybe_unused]] float dsc = 1.f, scale = 1.f;
-    if constexpr (NORM || DIG) {
-        float ss = 0.f, mx = 0.f;
+    if constexpr (NORM) {
+        float ss = 0.f;
 #pragma unroll
         for (int q = 0; q < XV; ++q)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                ss = fmaf(xin[q][e], xin[q][e], ss);
-                if constexpr (DIG) {
-                    const float t = fabsf(NORM ? xin[q][e] * nwin[q][e] : xin[q][e]);
-                    mx = t < INFINITY ? fmaxf(mx, t) : INFINITY;
-                }
-            }
-        if constexpr (NORM) ss = wave_sum(ss);
-        if constexpr (DIG) mx = wave_max(mx);
-        if (lane == 0) scratch[wave] = ss, scratch[4 + wave] = mx;
+            for (int e = 0; e < 4; ++e) ss = fmaf(xin[q][e], xin[q][e], ss);
+        ss = wave_sum(ss);
+        if (lane == 0) scratch[wave] = ss;
         __syncthreads();
-        if constexpr (NORM) {
-            ss = ((scratch[0] + scratch[1]) + scratch[2]) + scratch[3];
-            inv = rsqrtf(ss / static_cast<float>(a.cols) + a.eps);
-        }
-        if constexpr (DIG) {
-            mx = fmaxf(fmaxf(scratch[4], scratch[5]), fmaxf(scratch[6], scratch[7])) * inv;
-            const int e = wide_exponent<WT>(mx);
-            scale = ldexpf(1.f, e);
-            dsc = mx < INFINITY ? ldexpf(1.f, -e) : __builtin_nanf("");
-        }
-    }
-    if constexpr (NORM)
+        ss = ((scratch[0] + scratch[1]) + scratch[2]) + scratch[3];
+        const float inv = rsqrtf(ss / static_cast<float>(a.cols) + a.eps);
 #pragma unroll
         for (int q = 0; q < XV; ++q)
 #pragma unroll
             for (int e = 0; e < 4; ++e) xin[q][e] = xin[q][e] * inv * nwin[q][e];
+    }
     if constexpr (DIG) {
-        // Digit words of the thread's 8 columns in the weight words' layout.
+        // Digit words of the thread's 8 columns in the weight words' layout, with their chunk's scale.
         uint32_t* const xw = reinterpret_cast<uint32_t*>(xs[0]);
+        const float v8[8] = {xin[0][0], xin[0][1], xin[0][2], xin[0][3], xin[1][0], xin[1][1], xin[1][2], xin[1][3]};
+        const float scale = set_chunk_scale<WT>(v8, tid, chunk_scale);
         if constexpr (WT == WType::INT8) {
             const int at = (tid / 2 / kWave * XW * kWave + tid / 2 % kWave) * 4 + tid % 2 * 2;
 #pragma unroll
@@ -264,6 +268,10 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
     // The lane's inputs: digit words (int8 digit k of chunk c, word t (columns 4t .. 4t + 3) at dg[(2k + c) 4 + t]; int4
     // digit k of word t (columns 8t .. 8t + 7) at dg[4k + t]) or 32 floats and their sum.
     [[maybe_unused]] uint32_t dg[DIG ? 24 : 1];
+    [[maybe_unused]] float xscale[DIG ? F::CPL : 1];
+    if constexpr (DIG)
+#pragma unroll
+        for (int k = 0; k < F::CPL; ++k) xscale[k] = chunk_scale[k * kWave + lane];
     [[maybe_unused]] float xr[DIG ? 1 : NX], xsum = 0.f;
 #pragma unroll
     for (int k = 0; k < F::CPL; ++k)
@@ -292,21 +300,23 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
 #pragma unroll
         for (int i = 0; i < R; ++i) {
             if constexpr (DIG) {
-                // Per lane: int8 sum_k 256^k sum(q d_k); int4 sum_k 16^k sum(q d_k) (nibble u = q + 8, so q = u xor 8)
-                // times the lane's group scale.  The row's sum times 2^-e (and the int8 row scale at the store).
+                // Per chunk: int8 sum_k 256^k sum(q d_k); int4 sum_k 16^k sum(q d_k) (nibble u = q + 8, so q = u xor 8)
+                // times the lane's group scale; times the chunk's scale (and the row's sum times the int8 row scale at the store).
                 auto dot = [&](const u32x4* v, uint16_t g) {
                     if constexpr (WT == WType::INT8) {
-                        int a0 = 0, a1 = 0, a2 = 0;
+                        float sum = 0.f;
 #pragma unroll
-                        for (int c = 0; c < 2; ++c)
+                        for (int c = 0; c < 2; ++c) {
+                            int p[3] = {0, 0, 0};
 #pragma unroll
-                            for (int t = 0; t < 4; ++t) {
-                                const int w = static_cast<int>(v[c][t]);
-                                a0 = __builtin_amdgcn_sdot4(w, static_cast<int>(dg[(0 + c) * 4 + t]), a0, false);
-                                a1 = __builtin_amdgcn_sdot4(w, static_cast<int>(dg[(2 + c) * 4 + t]), a1, false);
-                                a2 = __builtin_amdgcn_sdot4(w, static_cast<int>(dg[(4 + c) * 4 + t]), a2, false);
-                            }
-                        return fmaf(fmaf(static_cast<float>(a2), 256.f, static_cast<float>(a1)), 256.f, static_cast<float>(a0));
+                            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                                for (int k = 0; k < 3; ++k)
+                                    p[k] = __builtin_amdgcn_sdot4(static_cast<int>(v[c][t]), static_cast<int>(dg[(2 * k + c) * 4 + t]), p[k], false);
+                            // p[0] + 256 p[1] stays below 2^27.
+                            sum = fmaf(fmaf(static_cast<float>(p[2]), 65536.f, static_cast<float>(p[0] + 256 * p[1])), xscale[c], sum);
+                        }
+                        return sum;
                     } else {
                         int ac[6] = {0, 0, 0, 0, 0, 0};
 #pragma unroll
@@ -316,7 +326,8 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
                             for (int k = 0; k < 6; ++k) ac[k] = __builtin_amdgcn_sdot8(w, static_cast<int>(dg[4 * k + t]), ac[k], false);
                         }
                         const int p0 = ac[0] + 16 * ac[1], p1 = ac[2] + 16 * ac[3], p2 = ac[4] + 16 * ac[5];
-                        return fmaf(static_cast<float>(p2), 65536.f, static_cast<float>(p0 + 256 * p1)) * half_bits_to_float(g);
+                        const float p = fmaf(static_cast<float>(p2), 65536.f, static_cast<float>(p0 + 256 * p1));
+                        return p * xscale[0] * half_bits_to_float(g);
                     }
                 };
                 d[i] = dot(b.v[i], b.g[i]);
@@ -341,7 +352,7 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
                 du[i] = su;
             }
         }
-        // Lane l: the sums of row r0 + (l mod R) (times 2^-e for the digit dots).  int4's 2048-wide rows (1 KiB, the
+        // Lane l: the sums of row r0 + (l mod R).  int4's 2048-wide rows (1 KiB, the
         // most rows per byte) reduce all R rows at once (rows_sum: int4 lm_head 28.2 -> 26.2 us, gate_up 8.0 -> 7.3 us
         // on MI355X); the other forms keep a full reduction per row, which measured as fast or faster for them (bf16
         // down 7.3 against 8.4 us).
@@ -360,11 +371,6 @@ __global__ void __launch_bounds__(kThreads) matvec_fast(MatvecArgs a) {
                 }
             }
         }
-        if constexpr (DIG) {
-            tot *= dsc;
-            tot_u *= dsc;
-        }
-
         if constexpr (KS == 1) {
             // Lane held + i keeps row r0 + i until the wave's last pass (no store inside the loop); held is a multiple
             // of R, so that lane already holds row i's sum.
@@ -579,18 +585,8 @@ __global__ void __launch_bounds__(kWideThreads) matvec_wide(MatvecArgs a, int un
             if constexpr (NORM) v[e] = v[e] * inv * nv[i][e / 4][e % 4];
         }
         uint32_t* const xw = reinterpret_cast<uint32_t*>(xs);
-        // The chunk's scale from its largest |x^| (infinite if one of them is infinite or NaN: its dots are NaN then).
         [[maybe_unused]] float scale = 1.f;
-        if constexpr (DIG) {
-            float m = 0.f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) m = fabsf(v[e]) < INFINITY ? fmaxf(m, fabsf(v[e])) : INFINITY;
-            m = fmaxf(m, dpp<kDppXor1>(m));
-            if constexpr (F::CPC == 32) m = fmaxf(m, dpp<kDppXor2>(m));
-            const int e = wide_exponent<WT>(m);
-            scale = ldexpf(1.f, e);
-            if (j % (F::CPC / 8) == 0) chunk_scale[j / (F::CPC / 8)] = m < INFINITY ? ldexpf(1.f, -e) : __builtin_nanf("");
-        }
+        if constexpr (DIG) scale = set_chunk_scale<WT>(v, j, chunk_scale);
         if constexpr (WT == WType::BF16) {
 #pragma unroll
             for (int q = 0; q < 2; ++q)

@@ -166,9 +166,9 @@ def test_matvec_wide_non_finite_input(wtype, norm, value):
 @pytest.mark.parametrize("wtype", ["int8", "int4"])
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("outlier", [1e3, 1e6])
-@pytest.mark.parametrize("rows,cols,epilogue", [(1001, 1024, "store"), (500, 5120, "add"), (300, 12288, "store"),
-                                                (4096, 8192, "swiglu")])
-def test_matvec_wide_outlier_input(wtype, norm, outlier, rows, cols, epilogue):
+@pytest.mark.parametrize("rows,cols,epilogue", [(1001, 1024, "store"), (700, 2048, "store"), (500, 5120, "add"),
+                                                (300, 12288, "store"), (4096, 8192, "swiglu")])
+def test_matvec_outlier_input(wtype, norm, outlier, rows, cols, epilogue):
     """One input far above the others that meets zero weights: it may cost the 16 (int8) or 32 (int4) inputs of its own
     chunk bits, and no others.  A chunk's fixed-point words have a step of at most 2 m / 7829350 for its largest input m,
     which leaves a row an error of sigma = that step / sqrt(12) times the 2-norm of the row's weights in the chunk.  Bound
@@ -211,6 +211,22 @@ def test_matvec_wide_outlier_input(wtype, norm, outlier, rows, cols, epilogue):
         bound = bound + 1e-6 * ref.abs()
     excess = ((y.double() - ref).abs() / bound).max().item()
     assert excess <= 1, f"{excess} times the bound"
+
+
+@pytest.mark.parametrize("wtype", ["bf16", "int8", "int4"])
+@pytest.mark.parametrize("cols", [2048, 3072])
+@pytest.mark.parametrize("size,weight", [(1e15, 1e25), (1e-18, 1e-24), (1e-18, 1e24), (0.0, 1.0)])
+def test_matvec_norm_weight_range(wtype, cols, size, weight):
+    """Inputs whose products with the norm weights leave the floats' range although the normalised inputs do not."""
+    rows, rng = 40, np.random.default_rng(cols)
+    w, s, w64 = _operands(wtype, rows, cols, 7)
+    x = (size * rng.standard_normal(cols)).astype(np.float32)
+    norm_w = (weight * rng.uniform(0.5, 1.5, cols)).astype(np.float32)
+    eps = 1e-5 if size == 0 else 0.0
+    y = E.kernel_matvec("opt", wtype, "store", 1, 0, w, s, x, norm_w, eps, None, rows, cols)
+    x64 = x.astype(np.float64)
+    ref = w64 @ (x64 / np.sqrt((x64 * x64).mean() + eps) * norm_w)
+    assert np.linalg.norm(y - ref) <= 1e-5 * np.linalg.norm(ref)
 
 
 def test_stream_read_timed_hook():
