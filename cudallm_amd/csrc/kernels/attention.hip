@@ -141,10 +141,15 @@ __device__ __forceinline__ uint32_t part_f16(float x, float y, int p) {
     const uint32_t h = take_f16(x, y), m = take_f16(x, y), l = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, y));
     return p == 0 ? h : p == 1 ? m : p == 2 ? l : 0u;
 }
+// Whether the three parts leave anything of them.
+__device__ __forceinline__ bool parts_lose(float x, float y) {
+    (void)take_f16(x, y), (void)take_f16(x, y), (void)take_f16(x, y);
+    return x != 0.f || y != 0.f;
+}
 
 // The running softmax of the wave: lane (n, g) holds, for head n / 4, the largest dot product m (starting at the lowest
 // float) and its share l of the weights 2^kLift exp(score - largest), and in o[b][i] the sums of part i of head g's weights
-// times column 4 n + b.  kLift puts the largest weight at 2^15, so that a weight has all its bits down to 2^-39 of that.
+// times column 4 n + b.  kLift puts the largest weight at 2^15, so that a weight has all its bits down to 2^-39 of that and counts down to 2^-61.
 // Weights come from differences of dot products, so they keep their meaning however large the scores are.
 constexpr float kLift = 15.f;
 struct Running {
@@ -340,15 +345,18 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
     const int begin = waves + static_cast<int>(more * wi / waves), end = waves + static_cast<int>(more * (wi + 1) / waves);
     Running st{-FLT_MAX, 0.f, {}};
     float m_dot = -FLT_MAX;  // st.m without the query's scale
+    bool plain = false;
     if (wi < tiles) {
         if (!early) load(A, wi);
         __builtin_amdgcn_sched_barrier(0);
-        // The query's fp16 parts: the head's largest |q| scaled to 2^14 .. 2^15.
+        // The query's fp16 parts: the head's largest |q| scaled to 2^14 .. 2^15.  Bits below 2^-46 of that are lost: 2^-61 of
+        // the largest, nothing in a score as long as that is below 2^16.  From there a column that meets zero keys can be so
+        // large that the others' bits count, and a wave that lost any does without the parts.
         float big = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) big = fmaxf(big, fabsf(qv[i / 8][i % 8]));
         big = max_lanes_xor<32>(max_lanes_xor<16>(big));
-        const int e = big > 0.f && big < INFINITY ? min(max(14 - ilogbf(big), -110), 110) : 0;
+        const int e = big > 0.f && big < INFINITY ? min(14 - ilogbf(big), 110) : 0;
         f16x8 qb[2];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -356,6 +364,10 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
 #pragma unroll
             for (int i = 0; i < 4; ++i) p[i] = part_f16(ldexpf(qv[s][2 * i], e), ldexpf(qv[s][2 * i + 1], e), n % 4);
             qb[s] = __builtin_bit_cast(f16x8, p);
+        }
+        if (__builtin_expect(__any(big >= 65536.f), 0)) {
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) plain = plain || parts_lose(ldexpf(qv[i / 8][i % 8], e), ldexpf(qv[i / 8][i % 8 + 1], e));
         }
         const float sc = ldexpf(kScore2, -e), ps = ldexpf(1.f, -11 * (n % 4));
         auto step = [&](const KvTile& kv, int tile) { attend(kv, qb, ps, sc, st, tile * kTile, n, g, ctx); };
@@ -388,7 +400,7 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
     if (g == 0 && n % 4 == 0) sml[w][n / 4][0] = m_dot, sml[w][n / 4][1] = st.l;
     // An infinity or NaN among the inputs (or a score past the floats) leaves one here, as its parts do not add up to it:
     // such a wave starts over with plain products.
-    if (__any(!(fabsf(m_dot) < INFINITY) || !(fabsf(st.l) < INFINITY) || !(fabsf((y[0] + y[1]) + (y[2] + y[3])) < INFINITY)))
+    if (__any(plain || !(fabsf(m_dot) < INFINITY) || !(fabsf(st.l) < INFINITY) || !(fabsf((y[0] + y[1]) + (y[2] + y[3])) < INFINITY)))
         attend_plain(q + kvh * kGroup * kHd, kc + static_cast<size_t>(kvh) * max_seq * kHd, vc + static_cast<size_t>(kvh) * max_seq * kHd,
                      wi, begin, end, ctx, lane, so[w], sml[w]);
     __syncthreads();

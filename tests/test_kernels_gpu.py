@@ -437,6 +437,35 @@ def test_attention_dynamic_range(case):
     assert (out.double().cpu() - ref).norm() <= 1e-4 * ref.norm()
 
 
+@pytest.mark.parametrize("case", ["top of the floats", "one column far above", "far apart"])
+def test_attention_query_range(case):
+    """Finite queries at the top of the floats with finite scores; query columns so far apart that the small ones fall
+    below what the fp16 parts of a head hold, beside zero keys under the large ones.  The bound of the test above; the
+    first case's scores differ by far more than their rounding, so its softmax picks one token."""
+    import torch
+    nkv, max_seq, ctx = 2, 2048, 1900
+    g = torch.Generator(device="cuda")
+    g.manual_seed(23)
+    q = torch.randn(nkv, 4, 64, generator=g, device="cuda")
+    k, v = (torch.randn(nkv, max_seq, 64, generator=g, device="cuda").half() for _ in range(2))
+    if case == "top of the floats":
+        q = (torch.rand(nkv, 4, 64, generator=g, device="cuda") + 0.1) * 3e38 * q.sign()
+        k *= 1e-4
+    elif case == "one column far above":
+        q[..., 5] = 2.0 ** 70
+        k[..., 5] = 0.0
+    else:
+        q[..., ::2] *= 2.0 ** 100
+        k[..., ::2] = 0.0
+    pos = torch.tensor([ctx - 1], dtype=torch.int32, device="cuda")
+    out = torch.empty(nkv * 256, device="cuda")
+    E.launch_attention_static(q.data_ptr(), k.data_ptr(), v.data_ptr(), pos.data_ptr(), out.data_ptr(), 4 * nkv, nkv, 64,
+                              max_seq, torch.cuda.current_stream().cuda_stream)
+    s = torch.matmul(q.double().cpu(), k[:, :ctx].double().cpu().transpose(1, 2)) * 0.125
+    ref = torch.matmul(torch.softmax(s, dim=-1), v[:, :ctx].double().cpu()).view(-1)
+    assert (out.double().cpu() - ref).norm() <= 1e-4 * ref.norm()
+
+
 @pytest.mark.parametrize("where", ["k", "v", "q"])
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
 def test_attention_non_finite(where, value):
