@@ -339,7 +339,8 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
     const bool early = split == 0 && (w + 1) * kTile <= max_seq;
     if (early) load(A, wi);
     const int ctx = *d_pos + 1;
-    const int tiles = (ctx + kTile - 1) / kTile, used = min(splits, (tiles + kWaves - 1) / kWaves), waves = kWaves * used;
+    // At least one split works, so that a position before the first token gives the sums' 0 / 0.
+    const int tiles = (ctx + kTile - 1) / kTile, used = max(1, min(splits, (tiles + kWaves - 1) / kWaves)), waves = kWaves * used;
     if (split >= used) return;
     const uint64_t more = max(tiles - waves, 0);
     const int begin = waves + static_cast<int>(more * wi / waves), end = waves + static_cast<int>(more * (wi + 1) / waves);

@@ -370,6 +370,19 @@ def test_attention_launch_splits(nkv, max_seq, shift):
         assert err <= 1e-5 * v.abs().max().item(), f"ctx {ctx}: {err}"
 
 
+@pytest.mark.parametrize("pos", [-1, -2, -300])
+def test_attention_without_tokens(pos):
+    """A position before the first token: no token weighs anything, and every output is the sums' 0 / 0."""
+    import torch
+    nkv, max_seq = 2, 1024
+    q, out = torch.ones(nkv * 256, device="cuda"), torch.ones(nkv * 256, device="cuda")
+    k, v = (torch.ones(nkv, max_seq, 64, device="cuda").half() for _ in range(2))
+    d_pos = torch.tensor([pos], dtype=torch.int32, device="cuda")
+    E.launch_attention_static(q.data_ptr(), k.data_ptr(), v.data_ptr(), d_pos.data_ptr(), out.data_ptr(), 4 * nkv, nkv, 64,
+                              max_seq, torch.cuda.current_stream().cuda_stream)
+    assert bool(out.isnan().all())
+
+
 def test_attention_replayed_launch():
     """A captured launch replayed over changing contexts (its split words are its own each time), against eager calls."""
     import torch
