@@ -155,10 +155,11 @@ __global__ void set_token_kernel(int* d_token, int token) { *d_token = token; }
 
 template <WType WT>
 __global__ void __launch_bounds__(256) embedding_kernel(const void* w, const void* scales, const int* d_token, float* x,
-                                                        int cols, int group) {
+                                                        int cols, int vocab, int group) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= cols) return;
-    const size_t tok = static_cast<size_t>(*d_token);
+    // The argmax of logits that are all NaN is no index of the vocabulary.
+    const size_t tok = static_cast<size_t>(min(max(*d_token, 0), vocab - 1));
     if constexpr (WT == WType::BF16) {
         x[j] = __builtin_bit_cast(float, static_cast<uint32_t>(static_cast<const uint16_t*>(w)[tok * cols + j]) << 16);
     } else if constexpr (WT == WType::INT8) {
@@ -284,15 +285,15 @@ void launch_embedding(WType wt, const void* w, const void* scales, const int* d_
     const dim3 grid((hidden + 255) / 256), block(256);
     switch (wt) {
         case WType::BF16:
-            hipLaunchKernelGGL(embedding_kernel<WType::BF16>, grid, block, 0, s, w, scales, d_token, x, hidden, group);
+            hipLaunchKernelGGL(embedding_kernel<WType::BF16>, grid, block, 0, s, w, scales, d_token, x, hidden, vocab, group);
             break;
         case WType::INT8:
             CLLM_REQUIRE(scales, "embedding: int8 needs scales");
-            hipLaunchKernelGGL(embedding_kernel<WType::INT8>, grid, block, 0, s, w, scales, d_token, x, hidden, group);
+            hipLaunchKernelGGL(embedding_kernel<WType::INT8>, grid, block, 0, s, w, scales, d_token, x, hidden, vocab, group);
             break;
         case WType::INT4:
             CLLM_REQUIRE(scales && group > 0 && hidden % group == 0 && hidden % 2 == 0, "embedding: int4 needs scales");
-            hipLaunchKernelGGL(embedding_kernel<WType::INT4>, grid, block, 0, s, w, scales, d_token, x, hidden, group);
+            hipLaunchKernelGGL(embedding_kernel<WType::INT4>, grid, block, 0, s, w, scales, d_token, x, hidden, vocab, group);
             break;
     }
     CLLM_HIP(hipGetLastError());

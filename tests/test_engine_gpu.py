@@ -6,11 +6,14 @@ bit-identical re-run after reset) on seeded synthetic Llama-3.2-1B-shaped files 
 model) instead of the HF checkpoint, plus graph-vs-eager identity, greedy decoding and state errors.
 """
 import os
+import shutil
 
 import numpy as np
 import pytest
 
 from cudallm_amd import engine as E
+from cudallm_amd import format as fmt
+from oracle import quantize as Q
 from oracle.model import OracleModel
 
 pytestmark = [pytest.mark.gpu, pytest.mark.timeout(900)]
@@ -96,6 +99,26 @@ def test_residuals(cfg, engine_runs, oracle_out):
             a, b = run["res"][p, k].astype(np.float64), ref[p, k].astype(np.float64)
             rel = np.linalg.norm(a - b) / np.linalg.norm(b)
             assert rel < 1e-3, f"position {p}, residual {k}: relative error {rel:.3e}"
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_token_after_nan_logits(model_path, tmp_path, graph):
+    """Logits that are all NaN have no argmax; a step that takes it as its token reads a row inside the embedding."""
+    path = tmp_path / "nan_norm.cudallm"
+    shutil.copyfile(model_path("int4"), path)
+    entries = {e["name"]: e for e in fmt.read_table(path)}
+    with open(path, "r+b") as f:
+        f.seek(entries["norm.weight"]["offset"])
+        f.write(np.full(2048, np.nan, np.float32).tobytes())
+    with E.Engine(path, fuse=False, cuda_graph=graph, max_seq_len=128) as eng:
+        assert eng.step_kind[0] == "program"
+        _, logits = eng.step(5, want_logits=True)
+        assert np.isnan(logits).all()
+        _, logits = eng.step(None, want_logits=True)
+        assert np.isnan(logits).all()
+        _, _, residuals = eng.step_debug(None)
+    packed, scales = (fmt.load_tensor(path, entries["tok_embeddings." + n]) for n in ("weight", "scales"))
+    np.testing.assert_allclose(residuals[0], Q.dequantize_int4_groups(packed[-1:], scales[-1:])[0], rtol=1e-6)
 
 
 @pytest.mark.parametrize("cfg", CONFIGS, ids=_id)
