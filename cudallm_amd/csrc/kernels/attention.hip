@@ -12,7 +12,9 @@
 #include <atomic>
 #include <cfloat>
 #include <mutex>
+#include <random>
 
+#include "../arrival.h"
 #include "../kernels.h"
 #include "device.h"
 
@@ -91,19 +93,17 @@ __global__ void __launch_bounds__(256) kv_write_kernel(const float* qkv, uint16_
 // whole query and the fp16 values the whole weight, with products exact and sums in 32 bits.  The weights come out of the
 // first product in the lanes in which the second takes them, eight tokens a lane.  About 180 instructions per tile, against
 // 480 with mixed-precision FMAs and a sum over lanes per score: that form measured, in one call of a replayed graph, 4.3 us
-// at 100 tokens, 10.7 at 8000 and 52.8 at 131071, this one 4.1, 9.9 and 46.
+// at 100 tokens, 10.7 at 8000 and 52.8 at 131071, this one 4.1, 10.0 and 46.5.
 //
 // A kv head's tiles are dealt evenly to its splits' waves, with only as many splits as give every wave a tile: up to 256
-// tokens are one workgroup, which writes the output.  With more, each split publishes its (o, m, l) as tagged words (value
-// and tag in one 64-bit word, so a word that carries the tag carries the value) and the last split's workgroup polls them
-// and writes the output: one store-to-load hop instead of a second launch.
-//  * The workgroups it waits for have smaller indices and wait for nothing, so they have been dispatched before it and
-//    always finish.  The wait is bounded besides; should it run out, the outputs are NaN.
-//  * The tag is a NaN pattern with the launch's number, which scratch memory does not hold by accident, and the words
-//    are zeroed as they are consumed, so a replayed launch (same number) never meets its own earlier words.
-// Measured on MI355X, 8 kv heads, one call in a replayed graph of 16 (2 at 131071), before (128 tokens per workgroup
-// staged in LDS, a second kernel merging the splits one after the other) and now: 100 tokens 6.5 -> 4.1 us, 1000
-// 9.7 -> 7.3, 4000 18.4 -> 8.4, 8000 28.0 -> 9.9, 131071 375 -> 46 (5.8 TB/s).
+// tokens are one workgroup, which writes the output.  With more, every split stores its (o, m, l), waits until they are in
+// memory and counts itself in the kv head's arrival word (arrival.h); the last to arrive merges them all, in split order
+// whichever it is, and writes the output.  No workgroup waits for another, so the order in which they run does not matter.
+// Polling for the partials instead (each word tagged, the last split's workgroup merging) measured 10.0 us at 8000 tokens
+// and 45 at 131071 against 8.9 and 44, and 6.7 against 6.85 at 300.
+// Measured on MI355X, 8 kv heads, one call in a replayed graph of 16 (2 at 131071), with 128 tokens per workgroup staged in
+// LDS and a second kernel merging the splits one after the other, and now: 100 tokens 6.5 -> 4.1 us, 1000 9.7 -> 7.1, 4000
+// 18.4 -> 8.1, 8000 28.0 -> 8.9, 131071 375 -> 44 (6.1 TB/s).
 // Workgroups in all: one per CU (2 waves per SIMD).  With the FMA form in workgroups of half the size, 512 measured 57
 // against 52 us at 131071 tokens and 12.7 against 11.4 at 8000, 128 measured 82 and 11.7.
 constexpr int kSplitBlocks = 256;
@@ -208,64 +208,62 @@ __device__ __forceinline__ void attend(const KvTile& kv, const f16x8 (&qb)[2], f
     }
 }
 
-// ---- tagged words -----------------------------------------------------------------------------------
+// ---- what the splits exchange ------------------------------------------------------------------------
 
-typedef __attribute__((address_space(1))) uint64_t global_u64;
-__device__ __forceinline__ uint64_t tag_load(const uint64_t* p) {
-    return __hip_atomic_load((global_u64*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Relaxed agent-scope accesses: they pass the XCDs' own L2 caches by and are made in the memory that all of them share.
+// Everything the splits exchange goes this way, so a store that has been acknowledged can be read anywhere, and a wave that
+// waits for its own stores needs no release fence, which would write back its whole L2 (8000 tokens 8.9 -> 16.0 us).
+template <typename T>
+using global_ptr = __attribute__((address_space(1))) T*;
+template <typename T>
+__device__ __forceinline__ T shared_load(const T* p) {
+    return __hip_atomic_load((global_ptr<T>)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void tag_store(uint64_t* p, float v, uint32_t tag) {
-    __hip_atomic_store((global_u64*)p, static_cast<uint64_t>(tag) << 32 | __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+template <typename T>
+__device__ __forceinline__ void shared_store(T* p, T v) {
+    __hip_atomic_store((global_ptr<T>)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ bool has_tag(uint64_t v, uint32_t tag) { return static_cast<uint32_t>(v >> 32) == tag; }
-__device__ __forceinline__ float value_of(uint64_t v) { return __builtin_bit_cast(float, static_cast<uint32_t>(v)); }
+// This wave's stores (and its begin()) have been made there.
+__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-constexpr unsigned kPollCap = 1u << 20;  // about a second
-
-// Where the partials of head h's split s lie: o as [h][s][64], then m and l as [h][s][2].
-struct Partials {
-    uint64_t *o, *ml;
-    uint32_t tag;
+struct ArrivalWord {  // arrival.h's operations
+    uint64_t* p;
+    __device__ void compare_exchange(uint64_t from, uint64_t to) const {
+        (void)__hip_atomic_compare_exchange_strong((global_ptr<uint64_t>)p, &from, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ uint64_t add_one() const {
+        return __hip_atomic_fetch_add((global_ptr<uint64_t>)p, uint64_t{1}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ void store(uint64_t v) const { shared_store(p, v); }
 };
 
-// The first n (<= used - 1) splits of head h that fall to this wave, s = half, half + 2, ...: their merged (m, l) and the
-// lane's output column.  Up to 16 of them, and all of their (m, l), are in flight at once.
+// Where the partials of head h's split s lie: o as [h][s][64], then m and l as [h][s][2]; each kv head's arrival word in a
+// 128-byte line of its own.
+constexpr int kWordStride = 16;
+struct Partials {
+    float *o, *ml;
+    uint64_t* words;
+    uint64_t tag;
+};
+
+// The splits of head h that fall to this wave, s = half, half + 2, ... below n: their merged (m, l) and the lane's output
+// column.  Up to 16 of them, and all of their (m, l), are in flight at once.
 __device__ __forceinline__ void merge_half(const Partials& p, int h, int splits, int n, int half, int lane, float& m, float& l,
                                            float& o) {
     constexpr int kRound = 16;
     m = -FLT_MAX, l = 0.f, o = 0.f;
-    uint64_t* po = p.o + static_cast<size_t>(h) * splits * kHd + lane;
-    uint64_t* pml = p.ml + static_cast<size_t>(h) * splits * 2;
-    const uint64_t none = static_cast<uint64_t>(p.tag) << 32;
+    const float* po = p.o + static_cast<size_t>(h) * splits * kHd + lane;
+    const float* pml = p.ml + static_cast<size_t>(h) * splits * 2;
     for (int s0 = half; s0 < n; s0 += 2 * kRound) {
-        const int sl = s0 + 2 * (lane % kRound);  // the split whose m (lanes 0-15) or l (16-31) this lane polls
+        const int sl = s0 + 2 * (lane % kRound);  // the split whose m (lanes 0-15) or l (16-31) this lane holds
         const bool mine = lane < 2 * kRound && sl < n;
-        uint64_t* const pm = pml + (mine ? 2 * sl + lane / kRound : 0);
-        uint64_t vm = mine ? tag_load(pm) : none, v[kRound];
+        const float vm = shared_load(pml + (mine ? 2 * sl + lane / kRound : 0));
+        float v[kRound];
 #pragma unroll
-        for (int i = 0; i < kRound; ++i) v[i] = s0 + 2 * i < n ? tag_load(po + static_cast<size_t>(s0 + 2 * i) * kHd) : none;
-        for (unsigned polls = 0;; ++polls) {
-            bool ok = has_tag(vm, p.tag);
-#pragma unroll
-            for (int i = 0; i < kRound; ++i) ok = ok && has_tag(v[i], p.tag);
-            if (__all(ok)) break;
-            if (polls == kPollCap) {
-                l = __builtin_nanf("");
-                return;
-            }
-            if (!has_tag(vm, p.tag)) vm = tag_load(pm);
-#pragma unroll
-            for (int i = 0; i < kRound; ++i)
-                if (!has_tag(v[i], p.tag)) v[i] = tag_load(po + static_cast<size_t>(s0 + 2 * i) * kHd);
-        }
-        // Consumed: zeroed for the next launch.
-        if (mine) tag_store(pm, 0.f, 0);
-#pragma unroll
-        for (int i = 0; i < kRound; ++i)
-            if (s0 + 2 * i < n) tag_store(po + static_cast<size_t>(s0 + 2 * i) * kHd, 0.f, 0);
-        const float sm = mine && lane < kRound ? value_of(vm) : -FLT_MAX;
-        const float sl_ = __shfl(value_of(vm), lane + kRound);
+        for (int i = 0; i < kRound; ++i) v[i] = shared_load(po + static_cast<size_t>(min(s0 + 2 * i, n - 1)) * kHd);
+        const float sm = mine && lane < kRound ? vm : -FLT_MAX;
+        const float sl_ = __shfl(vm, lane + kRound);
         const float mn = fmaxf(m, wave_max(sm)), f = weight_of(m, mn);
         const float e = mine && lane < kRound ? weight_of(sm, mn) : 0.f;
         m = mn;
@@ -273,7 +271,7 @@ __device__ __forceinline__ void merge_half(const Partials& p, int h, int splits,
         o *= f;
 #pragma unroll
         for (int i = 0; i < kRound; ++i)
-            if (s0 + 2 * i < n) o = fmaf(value_of(v[i]), __shfl(e, i), o);
+            if (s0 + 2 * i < n) o = fmaf(v[i], __shfl(e, i), o);
     }
 }
 
@@ -305,6 +303,7 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
                                                                    const int* d_pos, Partials part, float* out, int max_seq) {
     __shared__ float so[kWaves][kGroup][kHd];  // [wave][head][column]
     __shared__ float sml[kWaves][kGroup][2];   // [wave][head] m, l
+    __shared__ bool last;
 
     const int kvh = blockIdx.x, split = blockIdx.y, splits = gridDim.y;
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
@@ -342,6 +341,11 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
     // At least one split works, so that a position before the first token gives the sums' 0 / 0.
     const int tiles = (ctx + kTile - 1) / kTile, used = max(1, min(splits, (tiles + kWaves - 1) / kWaves)), waves = kWaves * used;
     if (split >= used) return;
+    // Every execution has its own tag: a replayed launch's packet lies elsewhere in the queue.
+    const ArrivalWord word{part.words + kvh * kWordStride};
+    const uint64_t tag = part.tag ^ reinterpret_cast<uint64_t>(__builtin_amdgcn_dispatch_ptr()) >> 6 << 8;
+    uint64_t seen = 0;
+    if (used > 1) seen = shared_load(word.p);
     const uint64_t more = max(tiles - waves, 0);
     const int begin = waves + static_cast<int>(more * wi / waves), end = waves + static_cast<int>(more * (wi + 1) / waves);
     Running st{-FLT_MAX, 0.f, {}};
@@ -406,10 +410,11 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
                      wi, begin, end, ctx, lane, so[w], sml[w]);
     __syncthreads();
 
+    if (used > 1 && tid == 0) arrival::begin(word, seen, tag);
     // Waves 0-3 take a head each: the 8 waves' partials in wave order.
     const int h = kvh * kGroup + w % kGroup;
-    float m = -FLT_MAX, l = 0.f, o = 0.f;
     if (w < kGroup) {
+        float m = -FLT_MAX, l = 0.f, o = 0.f;
 #pragma unroll
         for (int i = 0; i < kWaves; ++i) m = fmaxf(m, sml[i][w][0]);
 #pragma unroll
@@ -420,25 +425,31 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
         }
         if (used == 1) {
             out[h * kHd + lane] = o / l;
-        } else if (split + 1 < used) {
+        } else {
             const size_t slot = static_cast<size_t>(h) * splits + split;
-            tag_store(part.o + slot * kHd + lane, o, part.tag);
-            if (lane < 2) tag_store(part.ml + slot * 2 + lane, lane ? l : m, part.tag);
+            shared_store(part.o + slot * kHd + lane, o);
+            if (lane < 2) shared_store(part.ml + slot * 2 + lane, lane ? l : m);
+            stores_done();
         }
     }
-    if (split + 1 < used || used == 1) return;
+    if (used == 1) return;
 
-    // The last split: each head's other splits in two halves (waves w and w + 4), then the head's three partials.
-    float om, ol, oo;
-    merge_half(part, h, splits, used - 1, w / kGroup, lane, om, ol, oo);
-    __syncthreads();  // waves 0-3 have read so and sml
-    so[w][0][lane] = oo;
-    if (lane == 0) sml[w][0][0] = om, sml[w][0][1] = ol;
+    __syncthreads();
+    if (tid == 0) last = arrival::arrive(word, tag, used);
+    __syncthreads();
+    if (!last) return;
+    // Each head's splits in two halves (waves w and w + 4).
+    float m, l, o;
+    merge_half(part, h, splits, used, w / kGroup, lane, m, l, o);
+    if (w >= kGroup) {
+        so[w][0][lane] = o;
+        if (lane == 0) sml[w][0][0] = m, sml[w][0][1] = l;
+    }
     __syncthreads();
     if (w < kGroup) {
         const float m1 = sml[w + kGroup][0][0], l1 = sml[w + kGroup][0][1], o1 = so[w + kGroup][0][lane];
-        const float M = fmaxf(fmaxf(om, m1), m), f0 = weight_of(om, M), f1 = weight_of(m1, M), f = weight_of(m, M);
-        out[h * kHd + lane] = (oo * f0 + o1 * f1 + o * f) / (ol * f0 + l1 * f1 + l * f);
+        const float M = fmaxf(m, m1), f = weight_of(m, M), f1 = weight_of(m1, M);
+        out[h * kHd + lane] = (o * f + o1 * f1) / (l * f + l1 * f1);
     }
 }
 
@@ -520,12 +531,14 @@ void launch_attention_splitk(const float* q, const uint16_t* k_cache, const uint
     CLLM_REQUIRE(hd == kHd, "attention (split-K): needs head_dim 64");
     CLLM_REQUIRE(max_seq > 0 && max_seq % kAttnChunk == 0, "attention (split-K): max_seq must be a multiple of 128");
     CLLM_REQUIRE(aligned16(q) && aligned16(k_cache) && aligned16(v_cache), "attention: pointers must be 16-byte aligned");
-    // A word takes two of the caller's floats (and the first may lie one float further on, at 8 bytes).
-    const bool slack = (reinterpret_cast<uintptr_t>(part_o) | reinterpret_cast<uintptr_t>(part_ml)) & 7;
-    const int splits = std::max(1, std::min({(max_seq / kAttnChunk - slack) / 2, kSplitBlocks / nkv, kMaxSplits}));
-    auto words = [](float* p) { return reinterpret_cast<uint64_t*>((reinterpret_cast<uintptr_t>(p) + 7) & ~uintptr_t{7}); };
-    static std::atomic<uint32_t> launches{0};
-    const Partials part{words(part_o), words(part_ml), 0xFFC00000u | (launches.fetch_add(1, std::memory_order_relaxed) & 0x3FFFFFu)};
+    // Half of the caller's slots at most: the arrival words lie behind the outputs of the others.  (Two splits or more, the
+    // only ones that count, leave 8 slots of 64 floats for each kv head's line of 32.)
+    const int splits = std::max(1, std::min({max_seq / kAttnChunk / 2, kSplitBlocks / nkv, kMaxSplits}));
+    const auto end = reinterpret_cast<uintptr_t>(part_o + static_cast<size_t>(nh) * splits * kHd);
+    static const uint64_t salt = std::random_device{}() | static_cast<uint64_t>(std::random_device{}()) << 32;
+    static std::atomic<uint64_t> launches{0};
+    const Partials part{part_o, part_ml, reinterpret_cast<uint64_t*>((end + 7) & ~uintptr_t{7}),
+                        arrival::tag_of(salt, launches.fetch_add(1, std::memory_order_relaxed))};
     hipLaunchKernelGGL(attn_split_kernel, dim3(nkv, splits), dim3(kWaves * kWave), 0, s, q, k_cache, v_cache, d_pos, part, out,
                        max_seq);
     CLLM_HIP(hipGetLastError());
@@ -578,7 +591,7 @@ void launch_attention_splitk_static(const float* q, const uint16_t* k_cache, con
     CLLM_REQUIRE(static_cast<long long>(nh) * (max_seq / kAttnChunk) <= kStaticAttnSlots,
                  "attention (static scratch): nh * max_seq / 128 exceeds the 8192 partial slots of the static scratch");
     float* base = scratch_on_current_device();
-    // No clearing needed: a partial's words carry their launch's number, and the merge takes only words of its own launch.
+    // No clearing needed: the partials are written before they are read, and what the arrival words hold does not matter.
     launch_attention_splitk(q, k_cache, v_cache, d_pos, base, base + static_cast<size_t>(kStaticAttnSlots) * kHd, out,
                             nh, nkv, hd, max_seq, s);
 }

@@ -154,7 +154,8 @@ int cudallm_launch_matvec_timed(int weight_dtype, int epilogue, int rpb, const v
                                 const float* x, const float* norm_w, float eps, float* y, int rows, int cols,
                                 void* stream, void* start_event, void* stop_event);
 /* Split-K GQA attention over ctx = *d_pos + 1 tokens; part_o holds nh*(max_seq/128)*hd floats and
- * part_ml nh*(max_seq/128)*2 floats of scratch. */
+ * part_ml nh*(max_seq/128)*2 floats of scratch.  What the scratch holds before a call does not matter; calls that
+ * overlap need scratch of their own. */
 int cudallm_launch_attention(const float* q, const unsigned short* k_cache, const unsigned short* v_cache,
                              const int* d_pos, float* part_o, float* part_ml, float* out, int nh, int nkv, int hd,
                              int max_seq, void* stream);

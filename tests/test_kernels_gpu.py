@@ -370,6 +370,75 @@ def test_attention_launch_splits(nkv, max_seq, shift):
         assert err <= 1e-5 * v.abs().max().item(), f"ctx {ctx}: {err}"
 
 
+@pytest.mark.parametrize("fill", [0xFFC00000, 0xFFFFFFFF, 0x7FC00000, 0x3F800000, 0])
+def test_attention_scratch_content(fill):
+    """The caller's scratch may hold anything before a call, also before each replay of a captured one: NaNs, fills, and
+    what another shape's call left.  Bit for bit, since the splits are merged in their order whichever comes last."""
+    import torch
+    nkv, max_seq, ctx = 3, 4096, 4000
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    q = torch.randn(nkv * 256, generator=g, device="cuda")
+    k, v = (torch.randn(nkv, max_seq, 64, generator=g, device="cuda").half() for _ in range(2))
+    pos = torch.tensor([ctx - 1], dtype=torch.int32, device="cuda")
+    slots = 4 * nkv * (max_seq // 128)
+    part_o, part_ml = (torch.empty(slots * n, dtype=torch.int32, device="cuda") for n in (64, 2))
+    out, want = (torch.full((nkv * 256,), 9.0, device="cuda") for _ in range(2))
+    value = fill - (1 << 32) if fill >> 31 else fill
+
+    def launch(dst, kv_heads, seq):
+        E.launch_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), pos.data_ptr(), part_o.data_ptr(), part_ml.data_ptr(),
+                           dst.data_ptr(), 4 * kv_heads, kv_heads, 64, seq, torch.cuda.current_stream().cuda_stream)
+
+    part_o.fill_(value), part_ml.fill_(value)
+    launch(want, nkv, max_seq)
+    s = torch.matmul(q.double().view(nkv, 4, 64).cpu(), k[:, :ctx].double().cpu().transpose(1, 2)) * 0.125
+    ref = torch.matmul(torch.softmax(s, dim=-1), v[:, :ctx].double().cpu()).view(-1)
+    assert (want.double().cpu() - ref).abs().max().item() <= 1e-5 * v.abs().max().item()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        launch(out, nkv, max_seq)
+    for i in range(4):
+        out.fill_(9.0)
+        if i == 1:
+            part_o.fill_(value), part_ml.fill_(value)
+        elif i == 2:  # the other shape's words lie elsewhere
+            pos.fill_(2047), launch(out, 2, 2048), pos.fill_(ctx - 1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), f"replay {i}"
+
+
+@pytest.mark.parametrize("nkv", [3, 100])
+def test_attention_overlapping_calls(nkv):
+    """Calls on four streams at once, each stream with scratch of its own, give what they give one at a time."""
+    import torch
+    max_seq, n = 4096, 12
+    g = torch.Generator(device="cuda")
+    g.manual_seed(nkv)
+    k, v = (torch.randn(nkv, max_seq, 64, generator=g, device="cuda").half() for _ in range(2))
+    q = torch.randn(4 * n, nkv * 256, generator=g, device="cuda")
+    pos = torch.randint(0, max_seq, (4 * n,), generator=g, device="cuda", dtype=torch.int32)
+    slots = 4 * nkv * (max_seq // 128)
+    scratch = [(torch.empty(slots * 64, device="cuda"), torch.empty(slots * 2, device="cuda")) for _ in range(4)]
+    got, want = torch.zeros_like(q), torch.zeros_like(q)
+
+    def launch(i, out, stream):
+        part_o, part_ml = scratch[i % 4]
+        E.launch_attention(q[i].data_ptr(), k.data_ptr(), v.data_ptr(), pos[i].data_ptr(), part_o.data_ptr(),
+                           part_ml.data_ptr(), out[i].data_ptr(), 4 * nkv, nkv, 64, max_seq, stream.cuda_stream)
+
+    for i in range(4 * n):
+        launch(i, want, torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(4)]
+    for i in range(4 * n):
+        launch(i, got, streams[i % 4])
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("pos", [-1, -2, -300])
 def test_attention_without_tokens(pos):
     """A position before the first token: no token weighs anything, and every output is the sums' 0 / 0."""
@@ -489,7 +558,7 @@ def test_attention_non_finite(where, value):
     g.manual_seed(11)
     q = torch.rand(nkv * 256, generator=g, device="cuda") + 0.5
     k, v = (torch.randn(nkv, max_seq, 64, generator=g, device="cuda").half() for _ in range(2))
-    k[:, ctx:] = float("nan")  # past the context: never read
+    k[:, ctx:] = float("nan")  # past the context: read in whole tiles, but of no weight
     v[:, ctx:] = float("inf")
     if where == "q":
         q[d] = value
