@@ -80,11 +80,12 @@ def test_static_attention_replays_under_graph_capture_and_allocates_nothing(gpu)
         np.testing.assert_array_equal(out.cpu().numpy(), want, err_msg=f"graph replay {rep}")
     del g
     torch.cuda.synchronize()
-    free0 = torch.cuda.mem_get_info()[0]
     s = torch.cuda.current_stream().cuda_stream
-    for _ in range(4):
-        E.launch_attention_static(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr(), out.data_ptr(), nh, nkv,
-                                  64, max_seq, s)
-    torch.cuda.synchronize()
-    assert torch.cuda.mem_get_info()[0] == free0
+    for _ in range(2):  # the runtime may give the graph's memory back during the first calls: more free, not less
+        free0 = torch.cuda.mem_get_info()[0]
+        for _ in range(4):
+            E.launch_attention_static(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr(), out.data_ptr(), nh, nkv,
+                                      64, max_seq, s)
+        torch.cuda.synchronize()
+        assert torch.cuda.mem_get_info()[0] >= free0
     np.testing.assert_array_equal(out.cpu().numpy(), want)
