@@ -27,9 +27,8 @@
 //    2.82 -> 2.83 and 3.21 -> 3.26; 16384 x 2048 SWIGLU 5.23 -> 5.23 and 7.44 -> 7.49).  The 8192-wide down rows (KS = 4) keep the float path.
 //  * Row sums are wave64 DPP butterflies (deterministic order); with KS > 1 the slice partials
 //    meet in LDS and are added in slice order.  No atomics anywhere.
-//  * The grid: min(row blocks, CUs x the shape class's workgroups per CU (grid_per_cu; by default as
-//    many as can be resident)), but with KS = 1 at least enough workgroups that none takes more than
-//    64 / R passes.
+//  * The grid: min(row blocks, CUs x the shape class's workgroups per CU (grid_per_cu)), but with
+//    KS = 1 at least enough workgroups that none takes more than 64 / R passes.
 //
 // Widths other than 2048 and 8192 (and some of 8192, see pick_shape) use matvec_wide, which stages x in LDS.
 #pragma once
@@ -695,25 +694,14 @@ void dispatch(K kernel, int grid, int threads, size_t smem, hipStream_t s, const
     CLLM_HIP(hipGetLastError());
 }
 
-template <typename K>
-int resident_blocks(K kernel, size_t smem) {
-    int b = 0;
-    CLLM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, kernel, kThreads, smem));
-    CLLM_INTERNAL(b > 0, "matvec kernel cannot be resident");
-    return b;
-}
-
 template <WType WT, Epilogue EP, bool NORM, int KS, int R>
 void launch_fast(const MatvecArgs& a, hipStream_t s) {
     auto k = matvec_fast<WT, EP, NORM, KS, R>;
-    static const int occ = resident_blocks(k, 0);
     const int out_rows = EP == Epilogue::SWIGLU ? a.rows / 2 : a.rows;
     constexpr int ROWS_WG = (4 / KS) * R;
     const int need = (out_rows + ROWS_WG - 1) / ROWS_WG;
-    // Workgroups per CU: the shape class's choice, else as many as can be resident; but with KS = 1 no workgroup may
-    // take more than kMaxPasses<R> passes.
-    const int per_cu = grid_per_cu(WT, EP, a.rows, a.cols);
-    const int grid = std::max(std::min(need, device_cu_count() * (per_cu > 0 ? per_cu : occ)),
+    // The shape class's workgroups per CU; but with KS = 1 no workgroup may take more than kMaxPasses<R> passes.
+    const int grid = std::max(std::min(need, device_cu_count() * grid_per_cu(WT, EP, a.rows, a.cols)),
                               KS == 1 ? (need + kMaxPasses<R> - 1) / kMaxPasses<R> : 0);
     dispatch(k, grid, kThreads, 0, s, a);
 }

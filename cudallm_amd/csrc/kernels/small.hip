@@ -29,10 +29,11 @@ int device_cu_count() {
 // MI355X (each class's fastest mean kernel time).  Classes: 0 other (qkv, wo), 1 SwiGLU (gate_up), 2 8192 columns
 // (down), 3 vocabulary-sized (>= 65536 rows: lm_head).
 //
-// kDefaultRpb is the rpb used when the caller passes 0.  kGridPerCu caps the grid at that many workgroups per CU
-// (0: as many as can be resident at once).  Smaller grids mean fewer workgroups, each with more passes, so fewer
-// repeats of the input and norm prologue; larger ones than can be resident spread the last passes more evenly over
-// many rows, and the prologue of one workgroup runs under the loads of the others.  Measured, us:
+// kDefaultRpb is the rpb used when the caller passes 0.  kGridPerCu caps the grid at that many workgroups per CU.
+// Smaller grids mean fewer workgroups, each with more passes, so fewer repeats of the input and norm prologue; larger
+// ones than can be resident spread the last passes more evenly over many rows, and the prologue of one workgroup runs
+// under the loads of the others.  Measured, us (with one fixed-point scale per row; the scale per chunk that the
+// quantised types have now adds up to 2 %):
 //   bf16  qkv 4.69 -> 4.40, gate_up 12.50 -> 12.00 (1 per CU); 8192 columns 7.65 -> 7.50;
 //         128256 x 2048 81.7 (8 per CU) / 81.3 (16) / 80.0 (32) / 75.3 to 77.9 (one row block each); 256000 rows 158
 //         (16) / 146 to 152, 100000 rows 63.8 / 61.6
@@ -64,7 +65,8 @@ int type_index(WType wt) {
 }
 }  // namespace
 
-// The class's rpb, adjusted to the row count on 256 CUs:
+// The class's rpb, adjusted to the row count on 256 CUs (a device with fewer, a partition of this one say, gets the same
+// lines, which were not measured there):
 //  * Few rows of class 0 are spread over more workgroups: rpb is halved while they (4 waves of rpb rows each) would fill
 //    less than half of the CUs.  1500 x 2048: int8 3.06 -> 2.71 us, int4 2.83 -> 2.67; 512 rows: 2.89 -> 2.54, 2.77 -> 2.55.
 //  * Quantised rows of 8192 columns: each workgroup (rpb rows) reads 32 KiB of inputs, so rpb is doubled, up to 4 (int8) or

@@ -25,8 +25,7 @@ SHAPES = [("qkv", 3072, 2048, "store", True), ("wo", 2048, 2048, "add", False),
           ("lm_head", 128256, 2048, "store", True)]
 RPBS = (1, 2, 4, 8)
 # The library's choice when rpb = 0 (kDefaultRpb / default_rpb in csrc/kernels/small.hip), and its grid size in
-# workgroups per CU (kGridPerCu; 0: as many as can be resident), per weight type and shape class: other, SwiGLU, 8192
-# columns, >= 65536 rows.
+# workgroups per CU (kGridPerCu), per weight type and shape class: other, SwiGLU, 8192 columns, >= 65536 rows.
 DEFAULT_RPB = {"bf16": (1, 1, 2, 2), "int8": (4, 2, 2, 4), "int4": (4, 4, 4, 4)}
 GRID_PER_CU = {"bf16": (1, 1, 2, 1024), "int8": (2, 1, 2, 64), "int4": (2, 1, 2, 8)}
 
