@@ -138,7 +138,8 @@ __device__ __forceinline__ uint32_t take_f16(float& x, float& y) {
 // Part p of two floats written as h + m 2^-11 + l 2^-22 with fp16 h, m, l (p = 3: nothing): all 24 bits of a float between
 // 2^16 and 2^-24, and 2^-46 at the least, although fp16 itself ends at 2^-24.
 __device__ __forceinline__ uint32_t part_f16(float x, float y, int p) {
-    const uint32_t h = take_f16(x, y), m = take_f16(x, y), l = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, y));
+    const uint32_t h = take_f16(x, y), m = take_f16(x, y);
+    const uint32_t l = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, y));
     return p == 0 ? h : p == 1 ? m : p == 2 ? l : 0u;
 }
 // Whether the three parts leave anything of them.
@@ -149,7 +150,8 @@ __device__ __forceinline__ bool parts_lose(float x, float y) {
 
 // The running softmax of the wave: lane (n, g) holds, for head n / 4, the largest dot product m (starting at the lowest
 // float) and its share l of the weights 2^kLift exp(score - largest), and in o[b][i] the sums of part i of head g's weights
-// times column 4 n + b.  kLift puts the largest weight at 2^15, so that a weight has all its bits down to 2^-39 of that and counts down to 2^-61.
+// times column 4 n + b.  kLift puts the largest weight at 2^15, so that a weight has all its bits down to 2^-39 of
+// that and counts down to 2^-61.
 // Weights come from differences of dot products, so they keep their meaning however large the scores are.
 constexpr float kLift = 15.f;
 struct Running {
@@ -159,14 +161,16 @@ struct Running {
 
 // One tile at token t0; tokens at or past ctx weigh nothing.  qb: the group's queries, part n % 4 of head n / 4 as fp16 (one
 // power-of-two scale per head); ps: that part's scale; sc: the score scale times log2(e) over the head's scale.
-__device__ __forceinline__ void attend(const KvTile& kv, const f16x8 (&qb)[2], float ps, float sc, Running& st, int t0, int n, int g, int ctx) {
+__device__ __forceinline__ void attend(const KvTile& kv, const f16x8 (&qb)[2], float ps, float sc, Running& st, int t0, int n,
+                                       int g, int ctx) {
     // Scores of tokens 16 a + 4 g + i against (head, part) n; the parts' sum over the head's 4 lanes.
     f32x4 d[2];
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
         d[a] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int s = 0; s < 2; ++s) d[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, kv.k[a][s]), qb[s], d[a], 0, 0, 0);
+        for (int s = 0; s < 2; ++s)
+            d[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, kv.k[a][s]), qb[s], d[a], 0, 0, 0);
     }
     float x[8];
 #pragma unroll
@@ -203,8 +207,10 @@ __device__ __forceinline__ void attend(const KvTile& kv, const f16x8 (&qb)[2], f
     for (int b = 0; b < 4; ++b) {
         u32x4 c;  // column 4 n + b of the 8 tokens
 #pragma unroll
-        for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_perm(v[2 * i + 1][b / 2], v[2 * i][b / 2], b % 2 ? 0x07060302u : 0x05040100u);
-        st.o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, c), st.o[b], 0, 0, 0);
+        for (int i = 0; i < 4; ++i)
+            c[i] = __builtin_amdgcn_perm(v[2 * i + 1][b / 2], v[2 * i][b / 2], b % 2 ? 0x07060302u : 0x05040100u);
+        st.o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, c), st.o[b], 0,
+                                                         0, 0);
     }
 }
 
@@ -249,8 +255,8 @@ struct Partials {
 
 // The splits of head h that fall to this wave, s = half, half + 2, ... below n: their merged (m, l) and the lane's output
 // column.  Up to 16 of them, and all of their (m, l), are in flight at once.
-__device__ __forceinline__ void merge_half(const Partials& p, int h, int splits, int n, int half, int lane, float& m, float& l,
-                                           float& o) {
+__device__ __forceinline__ void merge_half(const Partials& p, int h, int splits, int n, int half, int lane, float& m,
+                                           float& l, float& o) {
     constexpr int kRound = 16;
     m = -FLT_MAX, l = 0.f, o = 0.f;
     const float* po = p.o + static_cast<size_t>(h) * splits * kHd + lane;
@@ -276,8 +282,8 @@ __device__ __forceinline__ void merge_half(const Partials& p, int h, int splits,
 }
 
 // The wave's tiles (`first`, then [begin, end)) one token at a time, lane = column: the closed form term by term.
-__device__ __forceinline__ void attend_plain(const float* q, const uint16_t* K, const uint16_t* V, int first, int begin, int end, int ctx,
-                                             int lane, float (&so)[kGroup][kHd], float (&sml)[kGroup][2]) {
+__device__ __forceinline__ void attend_plain(const float* q, const uint16_t* K, const uint16_t* V, int first, int begin,
+                                             int end, int ctx, int lane, float (&so)[kGroup][kHd], float (&sml)[kGroup][2]) {
 #pragma unroll 1
     for (int h = 0; h < kGroup; ++h) {
         const float qh = q[h * kHd + lane];
@@ -325,9 +331,11 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
 #pragma unroll
         for (int a = 0; a < 2; ++a)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) kv.k[a][s] = gload(reinterpret_cast<const u32x4*>(K + ko + a * 16 * kHd * 2 + s * 64));
+            for (int s = 0; s < 2; ++s)
+                kv.k[a][s] = gload(reinterpret_cast<const u32x4*>(K + ko + a * 16 * kHd * 2 + s * 64));
 #pragma unroll
-        for (int j = 0; j < 8; ++j) kv.v[j] = __builtin_nontemporal_load((const __attribute__((address_space(1))) u32x2*)(V + vo + token_of(0, j) * (kHd * 2)));
+        for (int j = 0; j < 8; ++j)
+            kv.v[j] = __builtin_nontemporal_load((global_ptr<const u32x2>)(V + vo + token_of(0, j) * (kHd * 2)));
     };
     // Wave wi takes tile wi and then its share of the tiles past one for each wave, in one piece (dealt in turn, 60 against
     // 53 us at 131071 tokens).  The first tile does not depend on *d_pos, so the first split's waves request theirs before
@@ -339,7 +347,8 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
     if (early) load(A, wi);
     const int ctx = *d_pos + 1;
     // At least one split works, so that a position before the first token gives the sums' 0 / 0.
-    const int tiles = (ctx + kTile - 1) / kTile, used = max(1, min(splits, (tiles + kWaves - 1) / kWaves)), waves = kWaves * used;
+    const int tiles = (ctx + kTile - 1) / kTile;
+    const int used = max(1, min(splits, (tiles + kWaves - 1) / kWaves)), waves = kWaves * used;
     if (split >= used) return;
     // Every execution has its own tag: a replayed launch's packet lies elsewhere in the queue.
     const ArrivalWord word{part.words + kvh * kWordStride};
@@ -354,9 +363,9 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
     if (wi < tiles) {
         if (!early) load(A, wi);
         __builtin_amdgcn_sched_barrier(0);
-        // The query's fp16 parts: the head's largest |q| scaled to 2^14 .. 2^15.  Bits below 2^-46 of that are lost: 2^-61 of
-        // the largest, nothing in a score as long as that is below 2^16.  From there a column that meets zero keys can be so
-        // large that the others' bits count, and a wave that lost any does without the parts.
+        // The query's fp16 parts: the head's largest |q| scaled to 2^14 .. 2^15.  Bits below 2^-46 are lost then: 2^-61 of
+        // the largest, nothing in a score as long as that is below 2^16.  From there a column that meets zero keys can be
+        // so large that the others' bits count, and a wave that lost any does without the parts.
         float big = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) big = fmaxf(big, fabsf(qv[i / 8][i % 8]));
@@ -372,7 +381,8 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
         }
         if (__builtin_expect(__any(big >= 65536.f), 0)) {
 #pragma unroll
-            for (int i = 0; i < 16; i += 2) plain = plain || parts_lose(ldexpf(qv[i / 8][i % 8], e), ldexpf(qv[i / 8][i % 8 + 1], e));
+            for (int i = 0; i < 16; i += 2)
+                plain = plain || parts_lose(ldexpf(qv[i / 8][i % 8], e), ldexpf(qv[i / 8][i % 8 + 1], e));
         }
         const float sc = ldexpf(kScore2, -e), ps = ldexpf(1.f, -11 * (n % 4));
         auto step = [&](const KvTile& kv, int tile) { attend(kv, qb, ps, sc, st, tile * kTile, n, g, ctx); };
@@ -405,9 +415,11 @@ __global__ void __launch_bounds__(kWaves* kWave) attn_split_kernel(const float* 
     if (g == 0 && n % 4 == 0) sml[w][n / 4][0] = m_dot, sml[w][n / 4][1] = st.l;
     // An infinity or NaN among the inputs (or a score past the floats) leaves one here, as its parts do not add up to it:
     // such a wave starts over with plain products.
-    if (__any(plain || !(fabsf(m_dot) < INFINITY) || !(fabsf(st.l) < INFINITY) || !(fabsf((y[0] + y[1]) + (y[2] + y[3])) < INFINITY)))
-        attend_plain(q + kvh * kGroup * kHd, kc + static_cast<size_t>(kvh) * max_seq * kHd, vc + static_cast<size_t>(kvh) * max_seq * kHd,
-                     wi, begin, end, ctx, lane, so[w], sml[w]);
+    auto finite = [](float v) { return fabsf(v) < INFINITY; };
+    if (__any(plain || !finite(m_dot) || !finite(st.l) || !finite((y[0] + y[1]) + (y[2] + y[3])))) {
+        const size_t head = static_cast<size_t>(kvh) * max_seq * kHd;
+        attend_plain(q + kvh * kGroup * kHd, kc + head, vc + head, wi, begin, end, ctx, lane, so[w], sml[w]);
+    }
     __syncthreads();
 
     if (used > 1 && tid == 0) arrival::begin(word, seen, tag);
