@@ -18,8 +18,8 @@
 //    and, with KS = 1, no store sits in the loop (each wave's row sums wait in its lanes until its last
 //    pass): either made the compiler's wait counts conservative, so that a pass also waited for the next
 //    pass's loads (128256 x 2048, bf16 82.5 -> 80.0 us, int8 44.6 -> 40.5,
-//    int4 32.2 -> 28.0).  With the launches of small.hip the same shape now takes 77.9, 41.4 and 23.7 us on
-//    MI355X: 6.7, 6.3 and 5.7 TB/s, where a plain stream read reaches 7.1.
+//    int4 32.2 -> 28.0).  With the launches of small.hip the same shape now takes 76.5, 39.5 and 23.2 us on
+//    MI355X: 6.9, 6.7 and 5.8 TB/s, where a plain stream read reaches 7.1.
 //  * Quantised 2048-wide rows (KS = 1) use integer digit dots: the workgroup turns the inputs into
 //    fixed-point digit words once (with a scale for each 16-byte chunk's columns), and a row then costs
 //    24 v_dot8_i32_i4 / v_dot4_i32_i8 per lane instead of a conversion and an FMA per column.  A scale per chunk
